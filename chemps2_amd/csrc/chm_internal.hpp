@@ -366,22 +366,39 @@ struct DevCopy {
   int pad;
 };
 
-// Thin SVD M = U diag(S) VT of one centre sector of Split by one-sided Jacobi. The
-// working matrix A (m x n, m >= n, column-major) is M, or M^T when M is wide; it is
-// overwritten. Q (n x n) is workspace. U is dLt x n and VT is n x dRt (leading
-// dimensions dLt and n), S descending.
+// Thin SVD M = U diag(S) VT of one centre sector of Split (svd.hip). A (m x n, m >= n,
+// column-major) is M, or M^T when M is wide; it is overwritten. U is dLt x n and VT is n x
+// dRt (leading dimensions dLt and n), S descending; the vectors of the n-long side that
+// belong to S = 0 come out as zeros (svd_complete fills them).
 struct DevSvd {
   double* A;
-  double* Q;
+  double* W;       // m x n workspace
+  double* X;       // n x n: R^T, then Ux Sigma
+  double* J;       // n x n: accumulated rotations
+  double* T;       // 256 per panel of 16 columns
   double* U;
   double* VT;
   double* S;
-  int* info;  // set to 1 when the sweeps end before every pair is orthogonal
+  double* floor2;  // norm^2 at or below which a column is numerically zero
+  int* perm;       // n
+  int* src;        // n
+  int* rot;        // SVD_SWEEPS: workgroups that rotated, by sweep (more than 32 columns)
+  int* info;       // 1 when the sweeps end before every pair is orthogonal (up to 32 columns)
   int m, n;
   int wide;
-  int max_sweeps;  // at most SVD_MAX_SWEEPS
+  int max_sweeps;  // at most SVD_SWEEPS
 };
-constexpr int SVD_JACOBI_MAXN = 256;  // largest n of the batched Jacobi kernel
+constexpr int SVD_SWEEPS = 40;      // sweep limit
+constexpr int SVD_ALONE = 32;       // sectors up to this width run all sweeps in one launch
+constexpr int SVD_MAXM = 1024;      // longest sector: a QR panel of 16 columns in LDS
+template <class T>
+struct DBuf;
+// Decomposes all jobs (sorted by falling n); buf holds their device copy. d_rot: the jobs'
+// counters, SVD_SWEEPS each, one after the other in any order; h_rot their host copy.
+void svd_batch(std::vector<DevSvd>& jobs, DBuf<DevSvd>& buf, int* h_rot, const int* d_rot, hipStream_t s);
+// Fills the n-long vectors of S = 0 so that the side is orthonormal (jobs as given to
+// svd_batch, whose buffers still hold).
+void svd_complete(std::vector<DevSvd>& jobs, DBuf<DevSvd>& buf, hipStream_t s);
 
 // Launchers (kernels.hip).
 // One dot product of two device arrays (the 2-RDM's P tensor with an operator).
@@ -394,7 +411,6 @@ struct DevDot {
 void launch_copies(const DevCopy* items, int n, hipStream_t s);
 // out[q] = a_q . b_q for every item q (one workgroup per item, fixed summation order)
 void launch_dots(const DevDot* items, int n, double* out, hipStream_t s);
-void launch_svd_jacobi(const DevSvd* items, int n, hipStream_t s);
 void launch_add_noise(double* x, int64_t n, uint64_t seed, double level, hipStream_t s);
 // mode 2: k_tiles_fit (matrix cores, only the 16 x 16 sub-tiles and k-steps that hold
 // elements), 1: k_tiles_mfma (matrix cores, whole 64 x 64 tiles), 0: k_tiles (vector FMA)

@@ -327,12 +327,22 @@ struct Ctx : HostState {
   static constexpr int SVD_STREAMS = 4;  // side streams of the large Split SVDs
   int64_t jacobi_retries = 0;            // Jacobi sectors decomposed again by rocSOLVER (not converged)
   int svd_max_sweeps = 0;                // CHM_SVD_MAX_SWEEPS: sweep limit of the Jacobi kernel (0: its own)
+  // Split's matrices and workspaces, kept between calls (grown as needed)
+  struct SplitWork {
+    DBuf<double> M, U, VT, S, E, W, X, J, T, F, jres;
+    DBuf<int> order, rot, info, jsw;
+    DBuf<DevCopy> items;
+    DBuf<DevSvd> jobs;
+    void release() {
+      for (DBuf<double>* b : {&M, &U, &VT, &S, &E, &W, &X, &J, &T, &F, &jres}) b->release();
+    }
+  } sw;
   std::vector<hipStream_t> svd_streams;
   std::vector<void*> svd_handles;
   std::vector<hipEvent_t> svd_ev_out;
   hipEvent_t svd_ev_in = nullptr;
   void side_streams(int n);
-  int svd_jacobi_maxn = SVD_JACOBI_MAXN;  // CHM_SVD_JACOBI_MAXN: larger centre sectors use rocSOLVER
+  int svd_jacobi_maxn = SVD_MAXM;  // CHM_SVD_JACOBI_MAXN: wider centre sectors use rocSOLVER
   double total_min = 1e8, max_disc_last = 0.0, last_min = 1e8;
   double tm[6] = {0, 0, 0, 0, 0, 0};  // seconds: join, prepare, davidson, split, update, total
   // Heff applications inside sweeps: F_H summed over applications and their device time
@@ -395,6 +405,7 @@ struct Ctx : HostState {
     bpart.release();
     W.release();
     u_arena.release();
+    sw.release();
     M_nnz = 0;
     site = -1;
   }

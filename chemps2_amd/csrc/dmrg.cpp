@@ -165,8 +165,8 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   struct Mult { int n, s, i, d; };
   struct Center {
     int nm, sm, im, dLt = 0, dRt = 0, cd = 0;
-    bool jac = false;  // batched Jacobi kernel (small sectors) or rocSOLVER
-    int64_t moff = 0, uoff = 0, voff = 0, soff = 0, qoff = 0;
+    bool jac = false;  // svd_batch or rocSOLVER (sectors longer than SVD_MAXM)
+    int64_t moff = 0, uoff = 0, voff = 0, soff = 0, qoff = 0, toff = 0;
     std::vector<Mult> lf, rt;
   };
   std::vector<Center> cs;
@@ -194,29 +194,43 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     c.cd = std::min(c.dLt, c.dRt);
     cs.push_back(c);
   }
-  int64_t msz = 0, usz = 0, vsz = 0, ssz = 0, qsz = 0;
+  int64_t msz = 0, usz = 0, vsz = 0, ssz = 0, qsz = 0, tsz = 0;
   for (auto& c : cs) {
     if (c.cd <= 0) continue;
-    c.jac = c.cd <= std::min(svd_jacobi_maxn, SVD_JACOBI_MAXN) && std::max(c.dLt, c.dRt) <= 4096;
+    c.jac = c.cd <= svd_jacobi_maxn && std::max(c.dLt, c.dRt) <= SVD_MAXM;
     c.moff = msz; msz += (int64_t)c.dLt * c.dRt;
     c.uoff = usz; usz += (int64_t)c.dLt * c.cd;
     c.voff = vsz; vsz += (int64_t)c.cd * c.dRt;
     c.soff = ssz; ssz += c.cd;
-    if (c.jac) { c.qoff = qsz; qsz += (int64_t)c.cd * c.cd; }
+    if (c.jac) {
+      c.qoff = qsz; qsz += (int64_t)c.cd * c.cd;
+      c.toff = tsz; tsz += (int64_t)(c.cd + 15) / 16 * 256;
+    }
   }
-  DBuf<double> M, U, VT, Sg, E, Qw;
-  Qw.alloc(std::max<int64_t>(qsz, 1));
+  // workspaces of svd_batch: the sorted matrices, X and J, the panels' T, floors, orders
+  // and sweep counters
+  DBuf<double>&M = sw.M, &U = sw.U, &VT = sw.VT, &Sg = sw.S, &E = sw.E, &Ww = sw.W, &Xw = sw.X, &Jw = sw.J, &Tw = sw.T, &Fw = sw.F;
+  DBuf<int>&Iw = sw.order, &Rw = sw.rot, &info = sw.info;
+  const int64_t nsec = (int64_t)cs.size();
+  Ww.alloc(std::max<int64_t>(qsz > 0 ? msz : 0, 1));
+  Xw.alloc(std::max<int64_t>(qsz, 1));
+  Jw.alloc(std::max<int64_t>(qsz, 1));
+  Tw.alloc(std::max<int64_t>(tsz, 1));
+  Fw.alloc(std::max<int64_t>(nsec, 1));
+  Iw.alloc(std::max<int64_t>(2 * ssz, 1));
+  Rw.alloc(std::max<int64_t>(nsec * SVD_SWEEPS, 1));
+  std::vector<int> h_rot(std::max<int64_t>(nsec * SVD_SWEEPS, 1), 0);
+  std::vector<DevSvd> jobs;  // of svd_batch
   M.alloc(std::max<int64_t>(msz, 1));
   U.alloc(std::max<int64_t>(usz, 1));
   VT.alloc(std::max<int64_t>(vsz, 1));
   Sg.alloc(std::max<int64_t>(ssz, 1));
   E.alloc(std::max<int64_t>(ssz, 1));
-  DBuf<rocblas_int> info;
   info.alloc(std::max<size_t>(cs.size(), 1));
   hip_check(hipMemsetAsync(info.p, 0, std::max<size_t>(cs.size(), 1) * sizeof(rocblas_int), stream), "clear info");
   // Assembly and SVD of the selected sectors (sel[q]): the centre matrices from the S
-  // blocks with their recoupling factors, then the batched Jacobi kernel for the small
-  // sectors and rocSOLVER for the others.
+  // blocks with their recoupling factors, then svd_batch for the sectors of at most
+  // SVD_MAXM rows and columns and rocSOLVER for the others.
   auto assemble_and_svd = [&](const std::vector<char>& sel) {
     std::vector<DevCopy> items;
     for (size_t q = 0; q < cs.size(); q++) {
@@ -231,7 +245,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
           const int fase = phase(a.s + b.s + s1 + s2);
           const int tjmin = std::max(std::abs(b.s - a.s), std::abs(s2 - s1)), tjmax = std::min(s1 + s2, a.s + b.s);
           DevCopy it{};
-          if (c.jac && c.dLt < c.dRt) {  // the Jacobi kernel works on M^T
+          if (c.jac && c.dLt < c.dRt) {  // svd_batch works on M^T
             it.dst = M.p + c.moff + ro + (int64_t)c.dRt * lo;
             it.ldd = c.dRt; it.trans = 1;
           } else {
@@ -258,28 +272,28 @@ double Ctx::split(int st, int D, bool mr, bool change) {
         lo += a.d;
       }
     }
-    DBuf<DevCopy> d_items;
-    d_items.upload(items, stream);
-    launch_copies(d_items.p, (int)items.size(), stream);
+    sw.items.upload(items, stream);
+    launch_copies(sw.items.p, (int)items.size(), stream);
     hip_check(hipGetLastError(), "split assembly");
-    std::vector<DevSvd> jobs;
+    std::vector<DevSvd> js;
     for (size_t q = 0; q < cs.size(); q++) {
       const auto& c = cs[q];
       if (c.cd > 0 && c.jac && sel[q]) {
         DevSvd j{};
-        j.A = M.p + c.moff; j.Q = Qw.p + c.qoff; j.U = U.p + c.uoff; j.VT = VT.p + c.voff; j.S = Sg.p + c.soff;
+        j.A = M.p + c.moff; j.W = Ww.p + c.moff; j.X = Xw.p + c.qoff; j.J = Jw.p + c.qoff; j.T = Tw.p + c.toff;
+        j.U = U.p + c.uoff; j.VT = VT.p + c.voff; j.S = Sg.p + c.soff;
+        j.floor2 = Fw.p + q; j.perm = Iw.p + 2 * c.soff; j.src = Iw.p + 2 * c.soff + c.cd;
         j.info = info.p + q;
         j.m = std::max(c.dLt, c.dRt); j.n = c.cd; j.wide = c.dLt < c.dRt;
-        j.max_sweeps = svd_max_sweeps;
-        jobs.push_back(j);
+        j.rot = Rw.p + (int64_t)SVD_SWEEPS * js.size();
+        j.max_sweeps = svd_max_sweeps > 0 ? std::min(svd_max_sweeps, SVD_SWEEPS) : SVD_SWEEPS;
+        js.push_back(j);
       }
     }
-    DBuf<DevSvd> d_jobs;
-    d_jobs.upload(jobs, stream);
-    launch_svd_jacobi(d_jobs.p, (int)jobs.size(), stream);
-    hip_check(hipGetLastError(), "split SVD kernel");
-    DBuf<double> jres;
-    DBuf<rocblas_int> jsw;
+    svd_batch(js, sw.jobs, h_rot.data(), Rw.p, stream);
+    if (!js.empty()) jobs = js;
+    DBuf<double>& jres = sw.jres;
+    DBuf<int>& jsw = sw.jsw;
     if (svd_large_gesvdj) {
       jres.alloc(std::max<size_t>(cs.size(), 1));
       jsw.alloc(std::max<size_t>(cs.size(), 1));
@@ -329,6 +343,8 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     copy_sync(stream, inf.data(), info.p, inf.size() * sizeof(rocblas_int), hipMemcpyDeviceToHost, "svd info");
     std::vector<char> redo(cs.size(), 0);
     bool any = false;
+    for (const DevSvd& j : jobs)  // wider sectors: the last sweep allowed still rotated
+      if (j.n > SVD_ALONE && h_rot[(j.rot - Rw.p) + j.max_sweeps - 1] != 0) inf[j.floor2 - Fw.p] = 1;
     for (size_t q = 0; q < cs.size(); q++) {
       if (inf[q] == 0) continue;
       if (!cs[q].jac) throw Error{ERR_NUMERIC, "SVD did not converge"};
@@ -388,6 +404,16 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     for (size_t i = 0; i < cs.size(); i++) v.push_back({cs[i].nm, cs[i].sm, cs[i].im, nd[i]});
     sec.set(st + 1, std::move(v));
   }
+  {
+    // vectors of zero singular values that are kept: completed to orthonormal sets
+    std::vector<DevSvd> zero;
+    for (const DevSvd& j : jobs) {
+      const Center& c = cs[j.floor2 - Fw.p];
+      const int lim = std::min(sec.dim(st + 1, c.nm, c.sm, c.im), c.cd);
+      if (c.jac && lim > 0 && sv[c.soff + lim - 1] == 0.0) zero.push_back(j);
+    }
+    svd_complete(zero, sw.jobs, stream);
+  }
   mps_alloc(st);
   mps_alloc(st + 1);
   if (mps[st].size > 0) hip_check(hipMemsetAsync(mps_buf[st], 0, mps[st].size * sizeof(double), stream), "clear");
@@ -423,9 +449,8 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     }
   }
   {
-    DBuf<DevCopy> d_items;
-    d_items.upload(items, stream);
-    launch_copies(d_items.p, (int)items.size(), stream);
+    sw.items.upload(items, stream);
+    launch_copies(sw.items.p, (int)items.size(), stream);
     hip_check(hipGetLastError(), "split scatter");
     hip_check(hipStreamSynchronize(stream), "split");
   }

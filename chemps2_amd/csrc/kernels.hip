@@ -1968,162 +1968,6 @@ __global__ __launch_bounds__(256) void k_copies(const DevCopy* __restrict__ item
   }
 }
 
-// One-sided (Hestenes) Jacobi SVD of the small centre-sector matrices of Split, one
-// workgroup of SVD_THREADS per matrix. Each round rotates a set of disjoint column pairs
-// (round-robin tournament order), every pair on a group of SVD_TPP lanes, all n / 2 pairs
-// of a round at once for n up to 2 SVD_GROUPS (one barrier per round); sweeps end when no pair
-// has |a_p . a_q| > sqrt(m) eps |a_p| |a_q|, the rounding floor of an m-term dot product
-// (the stopping rule of one-sided Jacobi in Drmac & Veselic, SIAM J. Matrix Anal. Appl.
-// 29 (2008) 1322, as LAPACK's dgesvj uses it). A job that reaches SVD_MAX_SWEEPS without
-// meeting it sets *info = 1. Columns whose norm is at most eps |A|_F are numerically zero:
-// they are not rotated (their directions are rounding noise and would keep the sweeps
-// going), their singular values are set to zero, and their vectors on the m-long side are
-// completed to an orthonormal set like those of exactly zero singular values.
-constexpr int SVD_THREADS = 1024;
-constexpr int SVD_TPP = 8;
-constexpr int SVD_GROUPS = SVD_THREADS / SVD_TPP;
-constexpr double SVD_EPS = 1.1102230246251565e-16;  // 2^-53
-constexpr int SVD_MAX_SWEEPS = 80;
-
-__device__ inline double group_sum(double v) {
-  for (int o = SVD_TPP / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, SVD_TPP);
-  return v;
-}
-
-__global__ __launch_bounds__(SVD_THREADS) void k_svd_jacobi(const DevSvd* __restrict__ items) {
-  const DevSvd it = items[blockIdx.x];
-  const int m = it.m, n = it.n;
-  const int tid = threadIdx.x, g = tid / SVD_TPP, l = tid % SVD_TPP;
-  double* A = it.A;
-  double* Q = it.Q;
-  __shared__ int rotated;
-  __shared__ double sig[SVD_JACOBI_MAXN];
-  __shared__ int src[SVD_JACOBI_MAXN];
-  __shared__ double fro[SVD_THREADS];
-  double f2 = 0.0;
-  for (int e = tid; e < m * n; e += SVD_THREADS) f2 += A[e] * A[e];
-  fro[tid] = f2;
-  for (int e = tid; e < n * n; e += SVD_THREADS) Q[e] = (e % n == e / n) ? 1.0 : 0.0;
-  __syncthreads();
-  for (int h = SVD_THREADS / 2; h > 0; h >>= 1) {
-    if (tid < h) fro[tid] += fro[tid + h];
-    __syncthreads();
-  }
-  const double floor2 = SVD_EPS * SVD_EPS * fro[0];
-  const int n2 = n + (n & 1);
-  const double tol = sqrt((double)m) * SVD_EPS;
-  bool converged = n <= 1;
-  const int max_sweeps = it.max_sweeps > 0 ? min(it.max_sweeps, SVD_MAX_SWEEPS) : SVD_MAX_SWEEPS;
-  for (int sweep = 0; sweep < max_sweeps && n > 1; sweep++) {
-    if (tid == 0) rotated = 0;
-    __syncthreads();
-    for (int r = 0; r < n2 - 1; r++) {
-      for (int k0 = 0; k0 < n2 / 2; k0 += SVD_GROUPS) {
-        const int k = k0 + g;
-        int p = -1, q = -1;
-        if (k < n2 / 2) {
-          p = (k == 0) ? 0 : ((k - 1 + r) % (n2 - 1)) + 1;
-          q = ((n2 - 2 - k + r) % (n2 - 1)) + 1;
-          if (p > q) { const int t = p; p = q; q = t; }
-          if (q >= n) p = q = -1;
-        }
-        double al = 0.0, be = 0.0, ga = 0.0;
-        if (p >= 0)
-          for (int i = l; i < m; i += SVD_TPP) {
-            const double x = A[i + (size_t)m * p], y = A[i + (size_t)m * q];
-            al += x * x; be += y * y; ga += x * y;
-          }
-        al = group_sum(al); be = group_sum(be); ga = group_sum(ga);
-        if (p >= 0 && ga != 0.0 && al > floor2 && be > floor2 && al > 0.0 && be > 0.0 && fabs(ga) > tol * sqrt(al * be)) {
-          const double zeta = (be - al) / (2.0 * ga);
-          const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-          const double c = 1.0 / sqrt(1.0 + t * t), s = c * t;
-          for (int i = l; i < m; i += SVD_TPP) {
-            const double x = A[i + (size_t)m * p], y = A[i + (size_t)m * q];
-            A[i + (size_t)m * p] = c * x - s * y;
-            A[i + (size_t)m * q] = s * x + c * y;
-          }
-          for (int i = l; i < n; i += SVD_TPP) {
-            const double x = Q[i + (size_t)n * p], y = Q[i + (size_t)n * q];
-            Q[i + (size_t)n * p] = c * x - s * y;
-            Q[i + (size_t)n * q] = s * x + c * y;
-          }
-          if (l == 0) rotated = 1;
-        }
-        __syncthreads();
-      }
-    }
-    __syncthreads();
-    const int any = rotated;
-    __syncthreads();
-    if (!any) {
-      converged = true;
-      break;
-    }
-  }
-  if (tid == 0 && it.info) *it.info = converged ? 0 : 1;
-  // singular values and their descending order
-  for (int j = g; j < n; j += SVD_GROUPS) {
-    double s2 = 0.0;
-    for (int i = l; i < m; i += SVD_TPP) s2 += A[i + (size_t)m * j] * A[i + (size_t)m * j];
-    s2 = group_sum(s2);
-    if (l == 0) sig[j] = s2 > floor2 ? sqrt(s2) : 0.0;
-  }
-  __syncthreads();
-  for (int j = tid; j < n; j += SVD_THREADS) {
-    int rank = 0;
-    for (int k = 0; k < n; k++) rank += (sig[k] > sig[j] || (sig[k] == sig[j] && k < j)) ? 1 : 0;
-    src[rank] = j;
-  }
-  __syncthreads();
-  // M = sum_j sig_j u_j v_j^T: u_j = a_j / sig_j and v_j = q_j (tall), or u_j = q_j and
-  // v_j = a_j / sig_j (wide, A = M^T)
-  const int ldU = it.wide ? n : m;
-  for (int t = g; t < n; t += SVD_GROUPS) {
-    const int j = src[t];
-    const double sj = sig[j];
-    const double inv = sj > 1e-250 ? 1.0 / sj : 0.0;
-    if (l == 0) it.S[t] = sj;
-    if (!it.wide) {
-      for (int i = l; i < m; i += SVD_TPP) it.U[i + (size_t)ldU * t] = A[i + (size_t)m * j] * inv;
-      for (int i = l; i < n; i += SVD_TPP) it.VT[t + (size_t)n * i] = Q[i + (size_t)n * j];
-    } else {
-      for (int i = l; i < n; i += SVD_TPP) it.U[i + (size_t)ldU * t] = Q[i + (size_t)n * j];
-      for (int i = l; i < m; i += SVD_TPP) it.VT[t + (size_t)n * i] = A[i + (size_t)m * j] * inv;
-    }
-  }
-  __syncthreads();
-  // vectors of (numerically) zero singular values: complete the m-long side to an
-  // orthonormal set by Gram-Schmidt on unit vectors (one wave, in order; every lane
-  // reads and writes only the elements i = lane (mod 64), lanes meet in shuffles)
-  if (tid < 64) {
-    for (int t = 0; t < n; t++) {
-      if (sig[src[t]] > 1e-250) continue;
-      double* base = it.wide ? it.VT : it.U;
-      const size_t rs = it.wide ? (size_t)n : 1;         // stride between elements
-      const size_t cs = it.wide ? 1 : (size_t)ldU;       // stride between vectors
-      for (int e = 0; e < m; e++) {
-        // v = e_e - sum_{t' < t} w_t' w_t'[e], accepted when |v| > 0.5
-        for (int i = tid; i < m; i += 64) base[i * rs + t * cs] = (i == e) ? 1.0 : 0.0;
-        for (int u = 0; u < t; u++) {
-          double d = 0.0;
-          for (int i = tid; i < m; i += 64) d += base[i * rs + u * cs] * base[i * rs + t * cs];
-          for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
-          for (int i = tid; i < m; i += 64) base[i * rs + t * cs] -= d * base[i * rs + u * cs];
-        }
-        double nn = 0.0;
-        for (int i = tid; i < m; i += 64) nn += base[i * rs + t * cs] * base[i * rs + t * cs];
-        for (int o = 32; o > 0; o >>= 1) nn += __shfl_xor(nn, o, 64);
-        if (nn > 0.25) {
-          const double f = 1.0 / sqrt(nn);
-          for (int i = tid; i < m; i += 64) base[i * rs + t * cs] *= f;
-          break;
-        }
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------- Davidson on the device ---
 // The scalars and small matrices of one Davidson solve (Davidson.cpp:105-191, 214-350) in
 // a DevDav record on the device; the kernels read the basis size from it, so the same
@@ -2670,10 +2514,6 @@ void launch_fill_hash(double* p, int64_t n, uint64_t seed, double scale, hipStre
 
 void launch_copies(const DevCopy* items, int n, hipStream_t s) {
   if (n > 0) hipLaunchKernelGGL(k_copies, dim3(n), dim3(256), 0, s, items);
-}
-
-void launch_svd_jacobi(const DevSvd* items, int n, hipStream_t s) {
-  if (n > 0) hipLaunchKernelGGL(k_svd_jacobi, dim3(n), dim3(SVD_THREADS), 0, s, items);
 }
 
 void launch_add_noise(double* x, int64_t n, uint64_t seed, double level, hipStream_t s) {
