@@ -738,135 +738,193 @@ void Ctx::prepare(int st) {
   }
   const double t_route = now_s();
   // ---- chained GEMM tiles for the remaining terms (in (out, in) order)
-  std::vector<DevGemmOp> o1;  // phase-1 products (host only: copied into the tile records)
+  // A two-operand term y += a op(L) x op(R) goes through W = op(L) x or W = x op(R). In a
+  // long list (tile_share_min two-operand terms) the order is the one of fewer
+  // multiplications, and terms of different output blocks with the same operator block and
+  // input share W (a carries over to phase 2): at the L = 32, D = 2000 middle site 1.60 M
+  // terms then have 1.23 M W of 4.4 GB instead of 1.60 M of 9.2 GB, and take 97 instead of
+  // 142 GF; 16.1 -> 12.6 ms a product. A short list keeps the reference's order and one W
+  // (with a) per term: launches and latency bound its product (402 against 382 us at 42 k
+  // terms, 383 against 362 us at 30 k), and its rounding stays that of the reference's order.
   DevTile1* t1 = nullptr;      // the device records, built in page-locked staging
   DevGemmOp* o2 = nullptr;
   DevTile* t2 = nullptr;
-  struct WRec { int64_t off; int rows, cols; };
-  std::vector<WRec> wrec(chain.size(), {-1, 0, 0});
+  auto two_op = [](const Term& t) { return t.tl != 'I' && t.tr != 'I'; };
+  int64_t ntwo = 0;
+  {
+    std::atomic<int64_t> sum{0};
+    parallel_for(((int64_t)chain.size() + 65535) / 65536, nthr, [&](int64_t c, int) {
+      int64_t n = 0;
+      for (size_t q = (size_t)c * 65536; q < std::min(chain.size(), (size_t)(c + 1) * 65536); q++) n += two_op(*chain[q]);
+      sum += n;
+    });
+    ntwo = sum;
+  }
+  const bool share = ntwo >= tile_share_min;
+  auto right_first = [&](const Term& t) {
+    if (!share) return t.xr_first;
+    const int64_t dL = dLof(t.out), dR = dRof(t.out), dLi = dLof(t.in), dRi = dRof(t.in);
+    return dL * dRi * (dLi + dR) > dLi * dR * (dRi + dL);
+  };
   auto rel_x = [&](int k) { return (const double*)(intptr_t)S.k2i[k]; };
   // The intermediates W of one batch of output blocks share the scratch buffer, so that
-  // it stays within a cap (one block larger than that is a batch of its own); apply()
-  // runs phase 1 and phase 2 batch after batch. The cap is tile_w_cap doubles if set,
-  // else a quarter of the free memory (the current buffer counted as free), at least
-  // 4 GiB.
+  // it stays within a cap (one block larger than that is a batch of its own; counted as if
+  // nothing were shared); apply() runs phase 1 and phase 2 batch after batch. The cap is
+  // tile_w_cap doubles if set, else a quarter of the free memory (the current buffer
+  // counted as free), at least 4 GiB.
   int64_t TILE_W_CAP = tile_w_cap;
   if (TILE_W_CAP <= 0) {
     size_t freeb = 0, totb = 0;
     hip_check(hipMemGetInfo(&freeb, &totb), "hipMemGetInfo");
     TILE_W_CAP = std::max<int64_t>((int64_t)1 << 29, (int64_t)((freeb + 8.0 * W.n) / 4 / 8));
   }
-  auto wneed = [&](const Term& t) -> int64_t {
-    if (t.tl == 'I' || t.tr == 'I') return 0;
-    const int dL = dLof(t.out), dR = dRof(t.out), dLi = dLof(t.in), dRi = dRof(t.in);
-    return t.xr_first ? ((int64_t)dLi * dR + 7) / 8 * 8 : ((int64_t)dL * dRi + 7) / 8 * 8;
+  struct WDim { int rows, cols; };
+  auto w_of = [&](const Term& t) -> WDim {
+    return right_first(t) ? WDim{dLof(t.in), dRof(t.out)} : WDim{dLof(t.out), dRof(t.in)};
   };
+  auto w_size = [](const WDim& w) { return ((int64_t)w.rows * w.cols + 7) / 8 * 8; };
+  const size_t nq = chain.size();
   std::vector<size_t> bstart;  // first chain index of every batch
-  int64_t Wmax = 0;
   {
+    // bytes of every output block on the host threads, then the batches
+    std::vector<std::pair<size_t, int64_t>> need;  // (first term, doubles) of an output block
+    const int64_t nc = ((int64_t)nq + 16383) / 16384;
+    std::vector<std::vector<std::pair<size_t, int64_t>>> part(nc);
+    parallel_for(nc, nthr, [&](int64_t c, int) {
+      const size_t q0 = (size_t)c * 16384, q1 = std::min(nq, q0 + 16384);
+      for (size_t q = q0; q < q1; q++) {
+        if (q == q0 || chain[q]->out != chain[q - 1]->out) part[c].push_back({q, 0});
+        if (two_op(*chain[q])) part[c].back().second += w_size(w_of(*chain[q]));
+      }
+    });
+    for (auto& v : part)
+      for (auto& e : v) {
+        if (!need.empty() && chain[need.back().first]->out == chain[e.first]->out) need.back().second += e.second;
+        else need.push_back(e);
+      }
     int64_t cur = 0;
-    for (size_t q0 = 0; q0 < chain.size();) {
-      size_t q1 = q0;
-      int64_t need = 0;
-      while (q1 < chain.size() && chain[q1]->out == chain[q0]->out) need += wneed(*chain[q1++]);
-      if (bstart.empty() || (cur > 0 && cur + need > TILE_W_CAP)) { bstart.push_back(q0); cur = 0; }
-      cur += need;
-      Wmax = std::max(Wmax, cur);
-      q0 = q1;
+    for (auto& e : need) {
+      if (bstart.empty() || (cur > 0 && cur + e.second > TILE_W_CAP)) { bstart.push_back(e.first); cur = 0; }
+      cur += e.second;
     }
   }
-  // Index pass: every two-operand term's phase-1 op and its W offset, and the phase-1
-  // tiles per batch and per bucket (tile_bucket), whose ranges tb1 holds as
-  // [B b + c, B b + c + 1) with B = TILE_BUCKETS. It runs on the host threads over chunks
-  // of terms that stay within one batch (counts, a prefix over the chunks, then the
-  // offsets); the records are filled the same way after the ops.
-  const size_t nq = chain.size();
-  std::vector<int> opi1(nq, -1);
+  const int nbatch = std::max<int>(1, (int)bstart.size());
   tb1.assign(1, 0);
   tb2.assign(1, 0);
   // tiles of 64 x 64 by bucket, or (wave_tiles) of 32 x 32, all on wavefronts
   const int ts1 = wave_tiles ? 32 : 64;
-  auto each_tile = [&](const WRec& w, auto&& f) {
+  auto each_tile = [&](const WDim& w, auto&& f) {
     for (int m0 = 0; m0 < w.rows; m0 += ts1)
       for (int n0 = 0; n0 < w.cols; n0 += ts1)
         f(m0, n0, wave_tiles ? 0 : tile_bucket(std::min(64, w.rows - m0), std::min(64, w.cols - n0)));
   };
-  auto w_of = [&](const Term& t) -> WRec {
-    return t.xr_first ? WRec{0, dLof(t.in), dRof(t.out)} : WRec{0, dLof(t.out), dRof(t.in)};
-  };
-  struct QChunk {
-    size_t q0, q1;
-    int batch;
-    int64_t ops = 0, w = 0;
+  // Per batch: the two-operand terms grouped by input block (a counting sort, stable), the
+  // distinct W of every group by a hash of the operator block, then W offsets and the
+  // phase-1 tiles per bucket (tile_bucket), whose ranges tb1 holds as [B b + c, B b + c + 1)
+  // with B = TILE_BUCKETS. Every position comes from prefix sums over the input blocks, so
+  // the lists do not depend on the thread count.
+  std::vector<int64_t> woff(nq, -1);    // W of every two-operand term
+  std::vector<uint32_t> wlist(nq);      // the terms by input block, batch after batch
+  struct InGrp {
+    size_t g0 = 0, g1 = 0;               // its terms in wlist
+    int64_t w = 0;                       // doubles of its distinct W, then their offset
     std::array<int64_t, TILE_BUCKETS> tiles{};
   };
-  std::vector<QChunk> qch;
-  const int nbatch = std::max<int>(1, (int)bstart.size());
-  for (int bt = 0; bt < nbatch; bt++) {
-    const size_t b0 = bstart.empty() ? 0 : bstart[bt], b1 = (bt + 1 < (int)bstart.size()) ? bstart[bt + 1] : nq;
-    for (size_t q = b0; q < b1; q += 8192) qch.push_back(QChunk{q, std::min(b1, q + 8192), bt});
-  }
-  parallel_for((int64_t)qch.size(), nthr, [&](int64_t ci, int) {
-    QChunk& C = qch[ci];
-    for (size_t q = C.q0; q < C.q1; q++) {
-      const Term& t = *chain[q];
-      if (t.tl == 'I' || t.tr == 'I') continue;
-      const WRec w = w_of(t);
-      C.ops++;
-      C.w += ((int64_t)w.rows * w.cols + 7) / 8 * 8;
-      each_tile(w, [&](int, int, int c) { C.tiles[c]++; });
+  std::vector<InGrp> ingrp((size_t)nbatch * nk);
+  std::vector<char> wfirst(nq, 0);      // the first term of every distinct W
+  int64_t Wmax = 0, nt1 = 0;
+  for (int bt = 0; bt < nbatch && nq > 0; bt++) {
+    const size_t b0 = bstart[bt], b1 = bt + 1 < nbatch ? bstart[bt + 1] : nq;
+    InGrp* G = ingrp.data() + (size_t)bt * nk;
+    const int R = (int)std::max<size_t>(1, std::min<size_t>(nthr, (b1 - b0 + 32767) / 32768));
+    std::vector<uint32_t> hist((size_t)R * nk, 0);
+    auto range = [&](int64_t r) { return std::make_pair(b0 + (b1 - b0) * r / R, b0 + (b1 - b0) * (r + 1) / R); };
+    parallel_for(R, nthr, [&](int64_t r, int) {
+      const auto rg = range(r);
+      for (size_t q = rg.first; q < rg.second; q++)
+        if (two_op(*chain[q])) hist[(size_t)r * nk + chain[q]->in]++;
+    });
+    size_t pos = b0;
+    for (int k = 0; k < nk; k++) {
+      G[k].g0 = pos;
+      for (int r = 0; r < R; r++) {
+        const uint32_t n = hist[(size_t)r * nk + k];
+        hist[(size_t)r * nk + k] = (uint32_t)pos;
+        pos += n;
+      }
+      G[k].g1 = pos;
     }
-  });
-  // prefix over the chunks: op index and W offset (per batch) at every chunk's start,
-  // tiles per batch and bucket
-  std::vector<int64_t> cops(qch.size()), cw(qch.size());
-  std::vector<std::array<int64_t, TILE_BUCKETS>> bcount(nbatch, std::array<int64_t, TILE_BUCKETS>{});
-  std::vector<std::array<int64_t, TILE_BUCKETS>> ctile(qch.size());
-  int no1 = 0;
-  {
-    int64_t ops = 0, wcur = 0;
-    int bt = -1;
-    for (size_t ci = 0; ci < qch.size(); ci++) {
-      if (qch[ci].batch != bt) { bt = qch[ci].batch; wcur = 0; }
-      cops[ci] = ops;
-      cw[ci] = wcur;
-      ops += qch[ci].ops;
-      wcur += qch[ci].w;
+    parallel_for(R, nthr, [&](int64_t r, int) {
+      const auto rg = range(r);
+      for (size_t q = rg.first; q < rg.second; q++)
+        if (two_op(*chain[q])) wlist[hist[(size_t)r * nk + chain[q]->in]++] = (uint32_t)q;
+    });
+    struct Key {
+      int64_t off;
+      int32_t buf, side;  // side: 1 left, 2 right operator first, + 4 when transposed
+    };
+    parallel_for(nk, nq < 16384 ? 1 : nthr, [&](int64_t k, int) {
+      InGrp& g = G[k];
+      const size_t n = g.g1 - g.g0;
+      if (n == 0) return;
+      size_t cap = 16;
+      while (cap < 2 * n) cap <<= 1;
+      std::vector<int> slot(cap, -1);    // index of a distinct W
+      std::vector<Key> keys;
+      std::vector<int64_t> offs;
+      for (size_t i = g.g0; i < g.g1; i++) {
+        const uint32_t q = wlist[i];
+        const Term& t = *chain[q];
+        const bool rf = right_first(t);
+        const Ref r = plan->ref(t, rf ? t.Rb : t.Lb);
+        const Key key{r.off, r.buf, (rf ? 2 : 1) + ((rf ? t.tr : t.tl) == 'T' ? 4 : 0)};
+        size_t h = FlatMap::mixh((uint64_t)key.off * 8 + key.side + ((uint64_t)key.buf << 40)) & (cap - 1);
+        while (slot[h] >= 0) {
+          const Key& o = keys[slot[h]];
+          if (share && o.off == key.off && o.buf == key.buf && o.side == key.side) break;
+          h = (h + 1) & (cap - 1);
+        }
+        if (slot[h] < 0) {
+          slot[h] = (int)keys.size();
+          keys.push_back(key);
+          offs.push_back(g.w);
+          const WDim w = w_of(t);
+          g.w += w_size(w);
+          wfirst[q] = 1;
+          each_tile(w, [&](int, int, int c) { g.tiles[c]++; });
+        }
+        woff[q] = offs[slot[h]];         // within the group
+      }
+    });
+    int64_t wcur = 0;
+    std::array<int64_t, TILE_BUCKETS> cnt{};
+    for (int k = 0; k < nk; k++) {
+      const int64_t w = G[k].w;
+      G[k].w = wcur;
+      wcur += w;
       for (int c = 0; c < TILE_BUCKETS; c++) {
-        ctile[ci][c] = bcount[bt][c];  // position within (batch, bucket), shifted below
-        bcount[bt][c] += qch[ci].tiles[c];
+        const int64_t n = G[k].tiles[c];
+        G[k].tiles[c] = cnt[c];
+        cnt[c] += n;
       }
     }
-    no1 = (int)ops;
-  }
-  int64_t nt1 = 0;
-  for (auto& bc : bcount)
+    Wmax = std::max(Wmax, wcur);
     for (int c = 0; c < TILE_BUCKETS; c++) {
-      nt1 += bc[c];
+      const int64_t base = nt1;
+      nt1 += cnt[c];
       tb1.push_back((int)std::min<int64_t>(nt1, INT32_MAX));
+      for (int k = 0; k < nk; k++) G[k].tiles[c] += base;
     }
-  for (size_t ci = 0; ci < qch.size(); ci++)
-    for (int c = 0; c < TILE_BUCKETS; c++) ctile[ci][c] += tb1[TILE_BUCKETS * qch[ci].batch + c];
-  parallel_for((int64_t)qch.size(), nthr, [&](int64_t ci, int) {
-    const QChunk& C = qch[ci];
-    int64_t op = cops[ci], wo = cw[ci];
-    for (size_t q = C.q0; q < C.q1; q++) {
-      const Term& t = *chain[q];
-      if (t.tl == 'I' || t.tr == 'I') continue;
-      WRec w = w_of(t);
-      w.off = wo;
-      wrec[q] = w;
-      wo += ((int64_t)w.rows * w.cols + 7) / 8 * 8;
-      opi1[q] = (int)op++;
-    }
-  });
+  }
+  if (nq == 0)
+    for (int c = 0; c < TILE_BUCKETS; c++) tb1.push_back(0);
   // Phase 2: an output block whose products are long (in 16-deep k chunks per tile) is
   // split into segments of consecutive products, so that the launch has many more
   // workgroups than the device holds at once; each segment writes its partial block into
   // the partial-sum buffer and k_chain_reduce adds them to y.
   auto chunks_of = [&](const Term& t) -> int64_t {
     if (t.tl == 'I' && t.tr == 'I') return 0;
-    const int k = (t.tr == 'I' || (t.tl != 'I' && t.xr_first)) ? dLof(t.in) : dRof(t.in);
+    const int k = (t.tr == 'I' || (t.tl != 'I' && right_first(t))) ? dLof(t.in) : dRof(t.in);
     return (k + 15) / 16;
   };
   // output blocks (the chained terms are in (out, in) order) and their work, on the host
@@ -988,45 +1046,37 @@ void Ctx::prepare(int st) {
   treds.upload(tred, stream);
   ntreds = (int)tred.size();
   W.alloc(std::max<int64_t>(Wmax, 1));
-  o1.resize(no1);
   tstage.reset();
   tstage.reserve(4 * 256 + nt1 * sizeof(DevTile1) + nq * sizeof(DevGemmOp) + nt2 * sizeof(DevTile));
   t1 = tstage.take<DevTile1>(nt1);
   o2 = tstage.take<DevGemmOp>(nq);
   t2 = tstage.take<DevTile>(nt2);
-  // phase 1: one group per two-operand term
-  parallel_for(((int64_t)nq + 4095) / 4096, nthr, [&](int64_t c, int) {
-    const size_t qe = std::min(nq, (size_t)(c + 1) * 4096);
-    for (size_t q = (size_t)c * 4096; q < qe; q++) {
-      if (opi1[q] < 0) continue;
+  // phase 1: the tiles of every distinct W
+  parallel_for(nq > 0 ? (int64_t)nbatch * nk : 0, nq < 16384 ? 1 : nthr, [&](int64_t gi, int) {
+    const InGrp& g = ingrp[gi];
+    std::array<int64_t, TILE_BUCKETS> pos = g.tiles;
+    for (size_t i = g.g0; i < g.g1; i++) {
+      const uint32_t q = wlist[i];
+      woff[q] += g.w;
+      if (!wfirst[q]) continue;
       const Term& t = *chain[q];
+      const WDim w = w_of(t);
       const int dL = dLof(t.out), dR = dRof(t.out), dLi = dLof(t.in), dRi = dRof(t.in);
-      DevGemmOp op{};
-      if (!t.xr_first) {
-        op.A = resolve(plan->ref(t, t.Lb)); op.lda = (t.tl == 'N') ? dL : dLi; op.ta = (t.tl == 'T');
-        op.B = rel_x(t.in); op.ldb = dLi; op.tb = 0; op.k = dLi; op.flags = 2;
+      DevTile1 tl{};
+      if (!right_first(t)) {
+        tl.A = resolve(plan->ref(t, t.Lb)); tl.lda = (t.tl == 'N') ? dL : dLi; tl.ta = (t.tl == 'T');
+        tl.B = rel_x(t.in); tl.ldb = dLi; tl.tb = 0; tl.k = dLi; tl.flags = 2;
       } else {
-        op.A = rel_x(t.in); op.lda = dLi; op.ta = 0;
-        op.B = resolve(plan->ref(t, t.Rb)); op.ldb = (t.tr == 'N') ? dRi : dR; op.tb = (t.tr == 'T'); op.k = dRi; op.flags = 1;
+        tl.A = rel_x(t.in); tl.lda = dLi; tl.ta = 0;
+        tl.B = resolve(plan->ref(t, t.Rb)); tl.ldb = (t.tr == 'N') ? dRi : dR; tl.tb = (t.tr == 'T'); tl.k = dRi;
+        tl.flags = 1;
       }
-      op.alpha = t.alpha;
-      op.kind = 0;
-      if (op.k <= 0) throw Error{ERR_STATE, "Heff plan: a phase-1 product with no inner dimension"};
-      o1[opi1[q]] = op;
-    }
-  });
-  parallel_for((int64_t)qch.size(), nthr, [&](int64_t ci, int) {
-    std::array<int64_t, TILE_BUCKETS> pos = ctile[ci];
-    for (size_t q = qch[ci].q0; q < qch[ci].q1; q++) {
-      if (opi1[q] < 0) continue;
-      const WRec& w = wrec[q];
-      const DevGemmOp& op = o1[opi1[q]];
+      if (tl.k <= 0) throw Error{ERR_STATE, "Heff plan: a phase-1 product with no inner dimension"};
+      tl.C = W.p + woff[q];
+      tl.alpha = share ? 1.0 : t.alpha;
+      tl.ldc = w.rows;
       each_tile(w, [&](int m0, int n0, int c) {
-        DevTile1 tl{};
-        tl.C = W.p + w.off;
-        tl.A = op.A; tl.B = op.B; tl.alpha = op.alpha;
-        tl.ldc = w.rows; tl.m0 = m0; tl.n0 = n0; tl.mrem = std::min(ts1, w.rows - m0); tl.nrem = std::min(ts1, w.cols - n0);
-        tl.lda = op.lda; tl.ldb = op.ldb; tl.k = op.k; tl.ta = op.ta; tl.tb = op.tb; tl.flags = op.flags;
+        tl.m0 = m0; tl.n0 = n0; tl.mrem = std::min(ts1, w.rows - m0); tl.nrem = std::min(ts1, w.cols - n0);
         t1[pos[c]++] = tl;
       });
     }
@@ -1050,16 +1100,14 @@ void Ctx::prepare(int st) {
       } else if (t.tl == 'I') {
         op.A = rel_x(t.in); op.lda = dLi; op.ta = 0;
         op.B = resolve(plan->ref(t, t.Rb)); op.ldb = (t.tr == 'N') ? dRi : dR; op.tb = (t.tr == 'T'); op.k = dRi; op.flags = 1;
-      } else if (!t.xr_first) {
-        const WRec& w = wrec[q];
-        op.alpha = 1.0;
-        op.A = W.p + w.off; op.lda = w.rows; op.ta = 0;
+      } else if (!right_first(t)) {
+        op.alpha = share ? t.alpha : 1.0;
+        op.A = W.p + woff[q]; op.lda = dL; op.ta = 0;
         op.B = resolve(plan->ref(t, t.Rb)); op.ldb = (t.tr == 'N') ? dRi : dR; op.tb = (t.tr == 'T'); op.k = dRi;
       } else {
-        const WRec& w = wrec[q];
-        op.alpha = 1.0;
+        op.alpha = share ? t.alpha : 1.0;
         op.A = resolve(plan->ref(t, t.Lb)); op.lda = (t.tl == 'N') ? dL : dLi; op.ta = (t.tl == 'T');
-        op.B = W.p + w.off; op.ldb = w.rows; op.tb = 0; op.k = dLi;
+        op.B = W.p + woff[q]; op.ldb = dLi; op.tb = 0; op.k = dLi;
       }
       o2[q] = op;
     }
@@ -2366,6 +2414,7 @@ int chm_ctx_create(int device, chm_ctx** out) {
   if (const char* e = std::getenv("CHM_CHAIN_ITEM_TERMS")) ctx->c.chain_item_terms = std::max(1, std::atoi(e));
   if (const char* e = std::getenv("CHM_CHAIN_GROUP_TERMS")) ctx->c.chain_group_terms = std::max(1, std::atoi(e));
   if (const char* e = std::getenv("CHM_SVD_GESVDJ")) ctx->c.svd_large_gesvdj = std::atoi(e) != 0;
+  if (const char* e = std::getenv("CHM_TILE_SHARE_MIN")) ctx->c.tile_share_min = std::atoll(e);
   if (const char* e = std::getenv("CHM_SVD_MAX_SWEEPS")) ctx->c.svd_max_sweeps = std::max(0, std::atoi(e));
   if (const char* e = std::getenv("CHM_TILE_W_CAP")) ctx->c.tile_w_cap = std::max(1LL, std::atoll(e));
   if (const char* e = std::getenv("CHM_OPS_KERNEL")) ctx->c.use_ops_kernel = std::atoi(e) != 0;

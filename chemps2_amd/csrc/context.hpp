@@ -151,6 +151,7 @@ struct Ctx : HostState {
   int tile_segments = 8192;   // CHM_TILE_SEGMENTS: phase-2 workgroups aimed at per launch
   int tile_seg_min = 64;      // CHM_TILE_SEG_MIN: fewest 16-deep k chunks per segment
   bool wave_tiles = false;    // CHM_WAVE_TILES=1: every tile 32 x 32 on one wavefront (no LDS sharing)
+  int64_t tile_share_min = 65536;  // CHM_TILE_SHARE_MIN: two-operand terms from which W are shared
   int64_t tile_w_cap = 0;  // doubles of W scratch per batch (CHM_TILE_W_CAP; 0: a quarter of free memory)
   DBuf<DevGemmOp> ops2;
   int ntiles1 = 0, ntiles2 = 0;

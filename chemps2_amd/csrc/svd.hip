@@ -294,10 +294,11 @@ __device__ __forceinline__ void times_rotations(double* X, double* J, int n, con
 
 // The rotation (c, s) that makes columns of norms^2 al, be and dot product ga orthogonal, or
 // the identity when |ga| <= tol sqrt(al be) (the rounding floor of the dot product, the
-// stopping rule of LAPACK's dgesvj) or a norm is at most the floor fl (numerically zero).
-// The tangent and the test come from the hardware's approximate reciprocal and roots
-// (about 26 bits: what is left of ga is that much smaller, which costs no sweep); the cosine
-// is refined to full precision, so the rotation is orthogonal whatever the tangent.
+// stopping rule of LAPACK's dgesvj) or a norm is at most the floor fl
+// (numerically zero). The tangent and the test come from the hardware's approximate
+// reciprocal and roots (about 26 bits: what is left of ga is that much smaller, which costs
+// no sweep); the cosine is refined to full precision, so the rotation is orthogonal whatever
+// the tangent.
 __device__ __forceinline__ void rotation(double al, double be, double ga, double tol, double fl, double& c, double& s) {
   const double d = be - al, h = __builtin_amdgcn_sqrt(fma(d, d, 4.0 * ga * ga));
   const double t = (d >= 0.0 ? 2.0 : -2.0) * ga * __builtin_amdgcn_rcp(fabs(d) + h);
