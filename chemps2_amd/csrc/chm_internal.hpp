@@ -243,6 +243,29 @@ struct DevTile1 {  // a tile of one GEMM product (k > 0, no axpy) with the produ
   int flags;  // bit 0: A relative to x, bit 1: B relative to x
   int pad;
 };
+// Phase-1 products of a long list, grouped by input block (k_strips): W = op(L) x or
+// x op(R) of one group of intermediates that share x. E: the operator block, element (j, k) at
+// E + sj j + sk k with j < len the row of op(L) or column of op(R) and k the inner index; O: W
+// (leading dimension ldc).
+struct DevStripW {
+  const double* E;
+  double* O;
+  int sj, sk, len, ldc;
+};
+struct DevXGroup {  // columns (left) or rows (right) [i0, i0 + ni) of x and W records [w0, w0 + nw)
+  int64_t xoff;     // input block in x, leading dimension ld
+  int ld, i0, ni, k;
+  int right, w0, nw, pad;
+};
+constexpr int STRIP_MAXK = 128;  // longest inner dimension of k_strips
+constexpr int STRIP_GROUP = 64;  // strips of 16 rows or columns per group, at most about
+constexpr int STRIP_BUCKETS = 24;
+// bucket of an inner dimension k and ni <= 64: 16-deep chunks of k (1, 2, 3, 4, 6 or 8) and
+// 16-wide tiles of ni
+inline int strip_bucket(int k, int ni) {
+  const int kc = (k + 15) / 16;
+  return (kc <= 4 ? kc - 1 : (kc <= 6 ? 4 : 5)) * 4 + (ni + 15) / 16 - 1;
+}
 constexpr int TILE_NO_AXPY = 4;  // no product of the tile is an axpy (kind 1)
 constexpr int TILE_C_PART = 8;   // C relative to the partial-sum buffer
 // Small-block products of the operator updates: one workgroup per work item computes
@@ -421,10 +444,12 @@ void launch_tiles(const DevTile* tiles, const DevGemmOp* ops, int ntiles, const 
 // wavefront per tile (k_tiles_wave1); c = 1..4, c sub-tiles per wavefront of a workgroup
 // per tile (k_tiles_stream1). The workgroups (TILE_STREAM_GROUPS, or TILE_WAVE_GROUPS of
 // four wavefronts for the wavefront buckets: what the device holds at once) walk the list.
-// Grouped tiles of at most 32 x 32 whose products are all GEMMs with k > 0: one
-// wavefront per tile (k_tiles_wave2).
-void launch_tiles_wave2(const DevTile* tiles, const DevGemmOp* ops, int ntiles, const double* xbase, double* ybase,
-                        hipStream_t s, double* pbase = nullptr);
+// Grouped tiles of at most 32 x 32: one wavefront per tile. shape: wave_shape of all of them, or
+// 3 (32 x 32) for any.
+void launch_tiles_wave2(const DevTile* tiles, const DevGemmOp* ops, int ntiles, int shape, const double* xbase,
+                        double* ybase, hipStream_t s, double* pbase = nullptr);
+constexpr int TILE2_RANGES = 5;  // four wave shapes and k_tiles_fit
+inline int wave_shape(int mrem, int nrem) { return (mrem > 16 ? 2 : 0) + (nrem > 16 ? 1 : 0); }
 constexpr int TILE_STREAM_GROUPS = 1024;
 constexpr int TILE_WAVE_GROUPS = 768;
 constexpr int TILE_BUCKETS = 7;
@@ -434,6 +459,9 @@ inline int tile_bucket(int mrem, int nrem) {
   if (mrem <= 16) return 6;
   return ((mrem + 15) / 16 * ((nrem + 15) / 16) + 3) / 4;
 }
+bool strip_kernel_setup();  // false: the device refuses the widest bucket's LDS
+void launch_strips(const DevXGroup* groups, int ngroups, const DevStripW* ws, int bucket, const double* xbase,
+                   hipStream_t s);
 void launch_tiles_stream1(const DevTile1* tiles, int ntiles, int c, const double* xbase, hipStream_t s);
 void launch_combos(const DevCombo* d_combos, const DevSrc* d_src, int ncombo, const int64_t* d_chunk_start,
                    int64_t nchunks, hipStream_t s);

@@ -829,10 +829,26 @@ void Ctx::prepare(int st) {
     size_t g0 = 0, g1 = 0;               // its terms in wlist
     int64_t w = 0;                       // doubles of its distinct W, then their offset
     std::array<int64_t, TILE_BUCKETS> tiles{};
+    // k_strips: distinct W by side (left, right operator) and their group chunks, then the
+    // first record of each side and the groups' first positions by bucket
+    int64_t nw[2] = {0, 0}, chunks[2] = {0, 0};
+    std::array<int32_t, STRIP_BUCKETS> xg{};
+  };
+  // A W goes to k_strips in a long list when its inner dimension fits, else to the tiles.
+  const bool use_strips = share && strips_ok;
+  // fewer strips per group in the shorter lists, so that the groups still fill the device
+  const int strip_group = (int)std::max<int64_t>(8, std::min<int64_t>(STRIP_GROUP, ntwo / 16384));
+  auto w_strip = [&](const Term& t, bool rf) { return use_strips && (rf ? dRof(t.in) : dLof(t.in)) <= STRIP_MAXK; };
+  // the groups of one side of an input block: chunks of about strip_group strips, for every
+  // 64 columns (left) or rows (right) of x
+  auto each_igroup = [&](int k, int side, auto&& f) {
+    const int ni = side ? dLof(k) : dRof(k), kin = side ? dRof(k) : dLof(k);
+    for (int i0 = 0; i0 < ni; i0 += 64) f(i0, std::min(64, ni - i0), kin, strip_bucket(kin, std::min(64, ni - i0)));
   };
   std::vector<InGrp> ingrp((size_t)nbatch * nk);
   std::vector<char> wfirst(nq, 0);      // the first term of every distinct W
-  int64_t Wmax = 0, nt1 = 0;
+  int64_t Wmax = 0, nt1 = 0, nstrip = 0, nxg = 0;
+  sb1.assign(1, 0);
   for (int bt = 0; bt < nbatch && nq > 0; bt++) {
     const size_t b0 = bstart[bt], b1 = bt + 1 < nbatch ? bstart[bt + 1] : nq;
     InGrp* G = ingrp.data() + (size_t)bt * nk;
@@ -872,6 +888,7 @@ void Ctx::prepare(int st) {
       std::vector<int> slot(cap, -1);    // index of a distinct W
       std::vector<Key> keys;
       std::vector<int64_t> offs;
+      int filled[2] = {strip_group, strip_group};  // strips in the current chunk of each side
       for (size_t i = g.g0; i < g.g1; i++) {
         const uint32_t q = wlist[i];
         const Term& t = *chain[q];
@@ -890,11 +907,20 @@ void Ctx::prepare(int st) {
           offs.push_back(g.w);
           const WDim w = w_of(t);
           g.w += w_size(w);
-          wfirst[q] = 1;
-          each_tile(w, [&](int, int, int c) { g.tiles[c]++; });
+          if (w_strip(t, rf)) {
+            wfirst[q] = 2;
+            if (filled[rf] >= strip_group) { g.chunks[rf]++; filled[rf] = 0; }
+            g.nw[rf]++;
+            filled[rf] += ((rf ? w.cols : w.rows) + 15) / 16;
+          } else {
+            wfirst[q] = 1;
+            each_tile(w, [&](int, int, int c) { g.tiles[c]++; });
+          }
         }
         woff[q] = offs[slot[h]];         // within the group
       }
+      for (int side = 0; side < 2; side++)
+        if (g.chunks[side] > 0) each_igroup((int)k, side, [&](int, int, int, int b) { g.xg[b] += (int)g.chunks[side]; });
     });
     int64_t wcur = 0;
     std::array<int64_t, TILE_BUCKETS> cnt{};
@@ -909,6 +935,20 @@ void Ctx::prepare(int st) {
       }
     }
     Wmax = std::max(Wmax, wcur);
+    for (int k = 0; k < nk; k++)
+      for (int side = 0; side < 2; side++) {
+        const int64_t n = G[k].nw[side];
+        G[k].nw[side] = nstrip;
+        nstrip += n;
+      }
+    for (int b = 0; b < STRIP_BUCKETS; b++) {
+      for (int k = 0; k < nk; k++) {
+        const int n = G[k].xg[b];
+        G[k].xg[b] = (int)nxg;
+        nxg += n;
+      }
+      sb1.push_back((int)std::min<int64_t>(nxg, INT32_MAX));
+    }
     for (int c = 0; c < TILE_BUCKETS; c++) {
       const int64_t base = nt1;
       nt1 += cnt[c];
@@ -916,8 +956,10 @@ void Ctx::prepare(int st) {
       for (int k = 0; k < nk; k++) G[k].tiles[c] += base;
     }
   }
-  if (nq == 0)
-    for (int c = 0; c < TILE_BUCKETS; c++) tb1.push_back(0);
+  if (nq == 0) {
+    tb1.resize(1 + TILE_BUCKETS, 0);
+    sb1.resize(1 + STRIP_BUCKETS, 0);
+  }
   // Phase 2: an output block whose products are long (in 16-deep k chunks per tile) is
   // split into segments of consecutive products, so that the launch has many more
   // workgroups than the device holds at once; each segment writes its partial block into
@@ -954,18 +996,35 @@ void Ctx::prepare(int st) {
   const int64_t nblk = (int64_t)bwork.size();
   std::vector<int> bseg(nblk, 1);
   {
-    int64_t wtot = 0;
+    // chunks of the blocks that fit a wavefront's 32 x 32, and of the others (per 64 x 64 tile)
+    int64_t wsmall = 0, wlarge = 0;
+    auto small = [&](int64_t bi) { return dLof(chain[bq[bi]]->out) <= 32 && dRof(chain[bq[bi]]->out) <= 32; };
     for (int64_t bi = 0; bi < nblk; bi++) {
       const int k = chain[bq[bi]]->out;
-      wtot += bwork[bi] * ((dLof(k) + 63) / 64) * ((dRof(k) + 63) / 64);
+      (small(bi) ? wsmall : wlarge) += bwork[bi] * ((dLof(k) + 63) / 64) * ((dRof(k) + 63) / 64);
     }
-    const int64_t wseg = std::max<int64_t>(std::max(1, tile_seg_min), wtot / std::max(1, tile_segments));
-    for (int64_t bi = 0; bi < nblk; bi++) bseg[bi] = (int)std::max<int64_t>(1, std::min<int64_t>(bwork[bi] / wseg, 64));
+    // segments of ws / wl chunks; returns the partial sums they need
+    auto cut = [&](int64_t ws, int64_t wl) {
+      int64_t part = 0;
+      for (int64_t bi = 0; bi < nblk; bi++) {
+        bseg[bi] = (int)std::max<int64_t>(1, std::min<int64_t>(bwork[bi] / std::max<int64_t>(std::max(1, tile_seg_min), small(bi) ? ws : wl), 64));
+        if (bseg[bi] > 1) part += (int64_t)bseg[bi] * dLof(chain[bq[bi]]->out) * dRof(chain[bq[bi]]->out);
+      }
+      return part;
+    };
+    // A long list gets enough segments of either kind to fill the device (a wavefront takes one
+    // of the small blocks': four times as many; 11.3 -> 10.6 ms a product at the L = 32, D = 2000
+    // middle site), unless their partial sums would near the static scratch of
+    // chm_heff_apply_noalloc; a short list one target over both.
+    const int64_t seg = std::max(1, tile_segments);
+    if (!share || cut(wsmall / (2 * seg), wlarge / seg) + bpart_need > ((int64_t)28 << 20))
+      cut((wsmall + wlarge) / seg, (wsmall + wlarge) / seg);
   }
   // Segment boundaries (about equal chunk counts) and whether a segment holds an axpy
-  // product, per block on the host threads; then the tiles per batch in two ranges,
-  // tb2[2 b] (tiles of at most 32 x 32 without axpy: one wavefront each, k_tiles_wave2)
-  // and tb2[2 b + 1] (the rest, k_tiles_fit).
+  // product, per block on the host threads; then the tiles per batch in TILE2_RANGES ranges of
+  // tb2: tiles of at most 32 x 32 on one wavefront each (k_tiles_wave2), by wave_shape in a
+  // long list (in a short one, where a launch is dear, all as 32 x 32), and the rest
+  // (k_tiles_fit).
   std::vector<int64_t> segq0(nblk + 1, 0);  // first segment of every block in segq / segax
   for (int64_t bi = 0; bi < nblk; bi++) segq0[bi + 1] = segq0[bi] + bseg[bi];
   std::vector<size_t> segq(segq0[nblk] + 1);  // first term of every segment
@@ -989,39 +1048,37 @@ void Ctx::prepare(int st) {
     }
   });
   segq[segq0[nblk]] = nq;
-  // the tiles of an output block (segment): 64 x 64, those of at most 32 x 32 without axpy
-  // on wavefronts; or (wave_tiles) 32 x 32 on wavefronts unless the segment has an axpy
+  // the tiles of an output block (segment): 64 x 64, those of at most 32 x 32 on wavefronts; or
+  // (wave_tiles) 32 x 32 on wavefronts unless the segment has an axpy
   auto each_tile2 = [&](int dL, int dR, bool ax, auto&& f) {
     const bool q32 = wave_tiles && !ax;
     const int st = q32 ? 32 : 64;
     for (int m0 = 0; m0 < dL; m0 += st)
-      for (int n0 = 0; n0 < dR; n0 += st)
-        f(m0, n0, q32 || (!ax && std::min(64, dL - m0) <= 32 && std::min(64, dR - n0) <= 32));
+      for (int n0 = 0; n0 < dR; n0 += st) {
+        const int mr = std::min(st, dL - m0), nr = std::min(st, dR - n0);
+        f(m0, n0, mr <= 32 && nr <= 32 ? (share ? wave_shape(mr, nr) : 3) : TILE2_RANGES - 1);
+      }
   };
-  std::vector<int64_t> tile2w(nblk), tile2f(nblk), bpart(nblk, -1);
+  std::vector<std::array<int64_t, TILE2_RANGES>> tile2(nblk);  // first tile of a block in every range
+  std::vector<int64_t> bpart(nblk, -1);
   int64_t nt2 = 0, tpart_n = 0;
   std::vector<DevBRed> tred;
   {
-    // per batch: wavefront tiles, then the rest
     size_t nextb = 1;
     int64_t bb = 0;  // first block of the batch
     auto close_batch = [&](int64_t be) {
-      int64_t nw = 0, nf = 0;
+      std::array<int64_t, TILE2_RANGES> n{};
       for (int64_t bi = bb; bi < be; bi++) {
         const int k = chain[bq[bi]]->out;
-        const int dL = dLof(k), dR = dRof(k);
-        int64_t cw = 0, cf = 0;
+        tile2[bi] = n;  // within the range, shifted below
         for (int64_t sgi = segq0[bi]; sgi < segq0[bi + 1]; sgi++)
-          each_tile2(dL, dR, segax[sgi] != 0, [&](int, int, bool wv) { (wv ? cw : cf)++; });
-        tile2w[bi] = nt2 + nw;
-        tile2f[bi] = nf;  // shifted below, once the batch's wavefront tiles are counted
-        nw += cw;
-        nf += cf;
+          each_tile2(dLof(k), dRof(k), segax[sgi] != 0, [&](int, int, int r) { n[r]++; });
       }
-      for (int64_t bi = bb; bi < be; bi++) tile2f[bi] += nt2 + nw;
-      tb2.push_back((int)(nt2 + nw));
-      nt2 += nw + nf;
-      tb2.push_back((int)nt2);
+      for (int r = 0; r < TILE2_RANGES; r++) {
+        for (int64_t bi = bb; bi < be; bi++) tile2[bi][r] += nt2;
+        nt2 += n[r];
+        tb2.push_back((int)std::min<int64_t>(nt2, INT32_MAX));
+      }
       bb = be;
     };
     for (int64_t bi = 0; bi < nblk; bi++) {
@@ -1039,7 +1096,7 @@ void Ctx::prepare(int st) {
     }
     close_batch(nblk);
   }
-  if (nt1 > INT32_MAX || nt2 > INT32_MAX || nq > (size_t)INT32_MAX) throw Error{ERR_SIZE, "too many Heff tiles"};
+  if (nt1 > INT32_MAX || nt2 > INT32_MAX || nstrip > INT32_MAX || nxg > INT32_MAX || nq > (size_t)INT32_MAX) throw Error{ERR_SIZE, "too many Heff tiles"};
   tpart_off = cpart_need;
   cpart_need += tpart_n;
   cpart.alloc(std::max<int64_t>(cpart_need, 1));
@@ -1047,14 +1104,32 @@ void Ctx::prepare(int st) {
   ntreds = (int)tred.size();
   W.alloc(std::max<int64_t>(Wmax, 1));
   tstage.reset();
-  tstage.reserve(4 * 256 + nt1 * sizeof(DevTile1) + nq * sizeof(DevGemmOp) + nt2 * sizeof(DevTile));
+  tstage.reserve(6 * 256 + nt1 * sizeof(DevTile1) + nq * sizeof(DevGemmOp) + nt2 * sizeof(DevTile) +
+                 nstrip * sizeof(DevStripW) + nxg * sizeof(DevXGroup));
+  DevStripW* sw1 = tstage.take<DevStripW>(nstrip);
+  DevXGroup* xg1 = tstage.take<DevXGroup>(nxg);
   t1 = tstage.take<DevTile1>(nt1);
   o2 = tstage.take<DevGemmOp>(nq);
   t2 = tstage.take<DevTile>(nt2);
-  // phase 1: the tiles of every distinct W
+  // phase 1: the strip records and groups, or the tiles, of every distinct W
   parallel_for(nq > 0 ? (int64_t)nbatch * nk : 0, nq < 16384 ? 1 : nthr, [&](int64_t gi, int) {
     const InGrp& g = ingrp[gi];
+    const int kin = (int)(gi % nk);
     std::array<int64_t, TILE_BUCKETS> pos = g.tiles;
+    std::array<int32_t, STRIP_BUCKETS> xpos = g.xg;
+    int64_t wpos[2] = {g.nw[0], g.nw[1]}, chunk0[2] = {g.nw[0], g.nw[1]};
+    int filled[2] = {0, 0};
+    auto close = [&](int side) {  // the chunk of W records collected last, for every i tile
+      if (wpos[side] == chunk0[side]) return;
+      each_igroup(kin, side, [&](int i0, int ni, int k, int b) {
+        DevXGroup x{};
+        x.xoff = S.k2i[kin]; x.ld = dLof(kin); x.i0 = i0; x.ni = ni; x.k = k; x.right = side;
+        x.w0 = (int)chunk0[side]; x.nw = (int)(wpos[side] - chunk0[side]);
+        xg1[xpos[b]++] = x;
+      });
+      chunk0[side] = wpos[side];
+      filled[side] = 0;
+    };
     for (size_t i = g.g0; i < g.g1; i++) {
       const uint32_t q = wlist[i];
       woff[q] += g.w;
@@ -1062,6 +1137,21 @@ void Ctx::prepare(int st) {
       const Term& t = *chain[q];
       const WDim w = w_of(t);
       const int dL = dLof(t.out), dR = dRof(t.out), dLi = dLof(t.in), dRi = dRof(t.in);
+      if (wfirst[q] == 2) {
+        const bool rf = right_first(t);
+        if (filled[rf] >= strip_group) close(rf);
+        DevStripW sw{};
+        sw.E = resolve(plan->ref(t, rf ? t.Rb : t.Lb));
+        sw.O = W.p + woff[q];
+        sw.len = rf ? dR : dL;
+        sw.ldc = w.rows;
+        // op(L)(j, k), j a row of dL, k of dLi; op(R)(k, j), k of dRi, j a column of dR
+        if (rf) { sw.sj = t.tr == 'N' ? dRi : 1; sw.sk = t.tr == 'N' ? 1 : dR; }
+        else { sw.sj = t.tl == 'N' ? 1 : dLi; sw.sk = t.tl == 'N' ? dL : 1; }
+        sw1[wpos[rf]++] = sw;
+        filled[rf] += (sw.len + 15) / 16;
+        continue;
+      }
       DevTile1 tl{};
       if (!right_first(t)) {
         tl.A = resolve(plan->ref(t, t.Lb)); tl.lda = (t.tl == 'N') ? dL : dLi; tl.ta = (t.tl == 'T');
@@ -1080,6 +1170,8 @@ void Ctx::prepare(int st) {
         t1[pos[c]++] = tl;
       });
     }
+    close(0);
+    close(1);
   });
   // phase 2: one group per output block (or per segment of it), added to the explicit
   // product
@@ -1113,12 +1205,12 @@ void Ctx::prepare(int st) {
     }
     // segments as the index pass cut them
     const int ns = bseg[bi];
-    int64_t tw = tile2w[bi], tf = tile2f[bi];
+    std::array<int64_t, TILE2_RANGES> pos = tile2[bi];
     for (int sg = 0; sg < ns; sg++) {
       const int64_t sgi = segq0[bi] + sg;
       const size_t qa = segq[sgi], qb = (sg == ns - 1) ? q1 : segq[sgi + 1];
       const bool axpy = segax[sgi] != 0;
-      each_tile2(dL, dR, axpy, [&](int m0, int n0, bool wv) {
+      each_tile2(dL, dR, axpy, [&](int m0, int n0, int r) {
           DevTile tl{};
           if (ns == 1) {
             tl.C = (double*)(intptr_t)S.k2i[k];
@@ -1129,7 +1221,7 @@ void Ctx::prepare(int st) {
           }
           if (!axpy) tl.flags |= TILE_NO_AXPY;
           tl.ldc = dL; tl.m0 = m0; tl.n0 = n0; tl.m = dL; tl.n = dR; tl.op0 = (int)qa; tl.nop = (int)(qb - qa);
-          t2[wv ? tw++ : tf++] = tl;
+          t2[pos[r]++] = tl;
         });
     }
   });
@@ -1140,9 +1232,11 @@ void Ctx::prepare(int st) {
     };
     up(ops2, o2, (int64_t)nq);
     up(tiles1, t1, nt1);
+    up(strips, sw1, nstrip);
+    up(xgroups, xg1, nxg);
     up(tiles2, t2, nt2);
   }
-  ntiles1 = (int)nt1;
+  ntiles1 = (int)(nt1 + nstrip);
   ntiles2 = (int)nt2;
   stats[6] = tot.pairs;
   stats[7] = (int64_t)chain.size() + stats[15];
@@ -1241,14 +1335,18 @@ void Ctx::apply_with(const double* xp, double* yp, double* bp, double* cp, doubl
   launch_bspmv(bitems.p, nbitems, breds.p, nbreds, bp, Mvals.p, M_nnz, M_split ? (mv_low ? 1 : 2) : 0, Mcol.p, xp,
                yp, stream);
   if (timing) hip_check(hipEventRecord(ev[1], stream), "event");
-  for (size_t b = 0; 2 * b + 2 < tb2.size(); b++) {  // GEMM tiles, batch by batch (W is shared)
+  for (size_t b = 0; TILE2_RANGES * (b + 1) < tb2.size(); b++) {  // GEMM tiles, batch by batch (W is shared)
+    for (int c = STRIP_BUCKETS - 1; c >= 0; c--) {
+      const int i = STRIP_BUCKETS * (int)b + c;
+      launch_strips(xgroups.p + sb1[i], sb1[i + 1] - sb1[i], strips.p, c, xp, stream);
+    }
     for (int c = 0; c < TILE_BUCKETS; c++) {
       const int i = TILE_BUCKETS * (int)b + c;
       launch_tiles_stream1(tiles1.p + tb1[i], tb1[i + 1] - tb1[i], c, xp, stream);
     }
-    const int w0 = tb2[2 * b], w1 = tb2[2 * b + 1], f1 = tb2[2 * b + 2];
-    launch_tiles_wave2(tiles2.p + w0, ops2.p, w1 - w0, xp, yp, stream, cp);
-    launch_tiles(tiles2.p + w1, ops2.p, f1 - w1, xp, yp, stream, tiles_kernel, cp);
+    const int* r = tb2.data() + TILE2_RANGES * b;
+    launch_tiles(tiles2.p + r[4], ops2.p, r[5] - r[4], xp, yp, stream, tiles_kernel, cp);
+    for (int q = 3; q >= 0; q--) launch_tiles_wave2(tiles2.p + r[q], ops2.p, r[q + 1] - r[q], q, xp, yp, stream, cp);
   }
   launch_chain_reduce(treds.p, ntreds, cp, yp, stream);  // segments of split output blocks
   if (timing) hip_check(hipEventRecord(ev[2], stream), "event");
@@ -2440,6 +2538,7 @@ int chm_ctx_create(int device, chm_ctx** out) {
     return CHM_ERR_HIP;
   }
   ctx->c.chain_large_ok = chm::chain_kernel_setup();
+  ctx->c.strips_ok = chm::strip_kernel_setup();
   ctx->c.fchain_ok = chm::fchain_kernel_setup();
   (void)hipGetLastError();
   if (!ctx->c.fchain_ok) ctx->c.use_fchain = false;

@@ -144,11 +144,15 @@ struct Ctx : HostState {
   DBuf<double> combo_arena, W, dx, dy, partial, scal;
   DBuf<DevTile1> tiles1;  // phase 1: W tiles of the two-operand terms, each with its product
   DBuf<DevTile> tiles2;
+  DBuf<DevStripW> strips;     // phase 1 of long lists: the W, grouped by input block (k_strips)
+  DBuf<DevXGroup> xgroups;
+  std::vector<int> sb1;       // group ranges per batch and bucket: [B b + c, B b + c + 1), B = STRIP_BUCKETS
+  bool strips_ok = false;     // the device grants k_strips its LDS
   std::vector<int> tb1, tb2;  // tile ranges of the batches that share the W scratch
   DBuf<DevBRed> treds;        // phase-2 output blocks split into segments: their reductions
   int ntreds = 0;
   int64_t tpart_off = 0;      // first partial sum of those segments in the chained partials
-  int tile_segments = 8192;   // CHM_TILE_SEGMENTS: phase-2 workgroups aimed at per launch
+  int tile_segments = 8192;    // CHM_TILE_SEGMENTS: phase-2 workgroups aimed at per launch
   int tile_seg_min = 64;      // CHM_TILE_SEG_MIN: fewest 16-deep k chunks per segment
   bool wave_tiles = false;    // CHM_WAVE_TILES=1: every tile 32 x 32 on one wavefront (no LDS sharing)
   int64_t tile_share_min = 65536;  // CHM_TILE_SHARE_MIN: two-operand terms from which W are shared

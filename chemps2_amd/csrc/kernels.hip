@@ -260,16 +260,54 @@ __global__ __launch_bounds__(NT) void k_tiles_mfma(const DevTile* __restrict__ t
 // The same tiles without the padding (k_tiles_fit): only the 16 x 16 sub-tiles that hold
 // elements of the block are computed, ms x ns of them (ms, ns <= 4), dealt out to the
 // four wavefronts in turn (wavefront w takes sub-tiles w, w + 4, ...; C = ceil(ms ns / 4)
-// per wavefront, a template argument so that every accumulator has a fixed register). The
-// staging is k_tiles_mfma's: two LDS buffers, the next chunk's operands loaded into
-// registers while the current one computes, one barrier per chunk. Tiles whose flags
-// carry TILE_NO_AXPY skip the search for axpy products; the others find them 64 records
-// at a time with a ballot.
+// per wavefront, a template argument so that every accumulator has a fixed register).
+// Chunks go through two LDS buffers with one barrier per chunk; the next chunk's operands
+// are in flight in registers while one computes. The record of the next product comes
+// in a product ahead as one vector load of a 32-bit word per lane (read with v_readlane
+// when due), so a product switch does not wait for a scalar load. The loads bound it: the
+// operands come from memory behind L2 for every product (10.5 GB at the L = 32, D = 2000 middle
+// site, in 3.8 ms).
+struct FitOp {
+  const double* A;
+  const double* B;
+  double alpha;
+  int lda, ldb, k, ta, tb;
+};
+// acc (16 x 16 sub-tiles at rows 16 si, columns 16 sj of the tile) += alpha * op(A) of every
+// axpy product of the tile, found 64 records at a time with a ballot
+template <int C>
+__device__ __forceinline__ void tile_axpys(chm_t4 (&acc)[C], const int (&si)[C], const int (&sj)[C], const bool (&on)[C],
+                                           const DevTile& t, const DevGemmOp* __restrict__ ops,
+                                           const double* __restrict__ xbase, int mrem, int nrem, int lane) {
+  const int lr = lane & 15, lg = lane >> 4;
+  for (int base = 0; base < t.nop; base += 64) {
+    const int oi = base + lane;
+    const int kind = oi < t.nop ? ops[t.op0 + oi].kind : 0;
+    uint64_t msk = __ballot(kind == 1);
+    while (msk) {
+      const int qb = __ffsll((unsigned long long)msk) - 1;
+      msk &= msk - 1;
+      const DevGemmOp op = ops[t.op0 + base + qb];
+      const double* A = rel(op.A, op.flags & 1, xbase);
+#pragma unroll
+      for (int q = 0; q < C; q++) {
+        if (!on[q]) continue;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int rr = 16 * si[q] + 4 * r + lg, cc = 16 * sj[q] + lr;
+          if (rr < mrem && cc < nrem)
+            acc[q][r] += op.alpha * (op.ta ? A[(size_t)(t.n0 + cc) + (size_t)op.lda * (t.m0 + rr)]
+                                           : A[(size_t)(t.m0 + rr) + (size_t)op.lda * (t.n0 + cc)]);
+        }
+      }
+    }
+  }
+}
 template <int C>
 __device__ __forceinline__ void tiles_fit_body(const DevTile& t, const DevGemmOp* __restrict__ ops,
                                                const double* __restrict__ xbase, double* __restrict__ ybase,
-                                               double* __restrict__ pbase,
-                                               double (*As)[TK][TM + 1], double (*Bs)[TK][TN + 1], int ms, int nsub) {
+                                               double* __restrict__ pbase, double (*As)[TK][TM + 1],
+                                               double (*Bs)[TK][TN + 1], int ms, int nsub) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -277,146 +315,6 @@ __device__ __forceinline__ void tiles_fit_body(const DevTile& t, const DevGemmOp
   // this wavefront's sub-tiles (q < C). A slot past nsub (only the last can be) repeats
   // a sub-tile of the block and is not stored, so that the MFMA sequence has no branch
   // (a conditional MFMA makes the compiler move the accumulators around it).
-  int si[C], sj[C];
-  bool on[C];
-#pragma unroll
-  for (int q = 0; q < C; q++) {
-    const int sq = wv + 4 * q;
-    on[q] = sq < nsub;
-    const int se = on[q] ? sq : 0;
-    si[q] = se % ms;
-    sj[q] = se / ms;
-  }
-  int offa[C], offb[C];
-#pragma unroll
-  for (int q = 0; q < C; q++) {
-    offa[q] = 16 * si[q] + lr;
-    offb[q] = 16 * sj[q] + lr;
-  }
-  chm_t4 acc[C];
-#pragma unroll
-  for (int q = 0; q < C; q++) acc[q] = chm_t4{0.0, 0.0, 0.0, 0.0};
-  // axpy products: C += alpha * op(A) on this lane's accumulator elements
-  if (!(t.flags & TILE_NO_AXPY)) {
-    for (int base = 0; base < t.nop; base += 64) {
-      const int oi = base + lane;
-      const int kind = oi < t.nop ? ops[t.op0 + oi].kind : 0;
-      uint64_t msk = __ballot(kind == 1);
-      while (msk) {
-        const int qb = __ffsll((unsigned long long)msk) - 1;
-        msk &= msk - 1;
-        const DevGemmOp op = ops[t.op0 + base + qb];
-        const double* A = rel(op.A, op.flags & 1, xbase);
-#pragma unroll
-        for (int q = 0; q < C; q++) {
-          if (!on[q]) continue;
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int rr = 16 * si[q] + 4 * r + lg, cc = 16 * sj[q] + lr;
-            if (rr < mrem && cc < nrem)
-              acc[q][r] += op.alpha * (op.ta ? A[(size_t)(t.n0 + cc) + (size_t)op.lda * (t.m0 + rr)]
-                                             : A[(size_t)(t.m0 + rr) + (size_t)op.lda * (t.n0 + cc)]);
-          }
-        }
-      }
-    }
-  }
-  int o = 0, k0 = 0;
-  auto skip = [&]() {  // advance o to the next GEMM product with work left
-    while (o < t.nop && (ops[t.op0 + o].kind == 1 || k0 >= ops[t.op0 + o].k)) { o++; k0 = 0; }
-  };
-  skip();
-  double ra[4], rb[4];
-  // this thread's elements of chunk (op, k0): (r, kk) of op(A), (kb, c) of op(B)
-  auto a_at = [&](const DevGemmOp& op, int q, int& r, int& kk) {
-    if (op.ta == 0) { r = tid & 63; kk = (tid >> 6) + 4 * q; } else { kk = tid & 15; r = (tid >> 4) + 16 * q; }
-  };
-  auto b_at = [&](const DevGemmOp& op, int q, int& kb, int& c) {
-    if (op.tb == 0) { kb = tid & 15; c = (tid >> 4) + 16 * q; } else { c = tid & 63; kb = (tid >> 6) + 4 * q; }
-  };
-  // raw global (not flat) loads only, a lane outside the block reading the block's first
-  // element: put applies the masks and alpha, so nothing here waits for the loads and the
-  // LDS waits of the compute do not wait for them either
-  auto fetch = [&]() {
-    const DevGemmOp op = ops[t.op0 + o];
-    gdbl* A = (gdbl*)rel(op.A, op.flags & 1, xbase);
-    gdbl* B = (gdbl*)rel(op.B, (op.flags >> 1) & 1, xbase);
-    const int krem = min(TK, op.k - k0);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      int r, kk, kb, c;
-      a_at(op, q, r, kk);
-      b_at(op, q, kb, c);
-      const size_t ia = op.ta ? (size_t)(k0 + kk) + (size_t)op.lda * (t.m0 + r) : (size_t)(t.m0 + r) + (size_t)op.lda * (k0 + kk);
-      const size_t ib = op.tb ? (size_t)(t.n0 + c) + (size_t)op.ldb * (k0 + kb) : (size_t)(k0 + kb) + (size_t)op.ldb * (t.n0 + c);
-      ra[q] = A[(r < mrem && kk < krem) ? ia : 0];
-      rb[q] = B[(c < nrem && kb < krem) ? ib : 0];
-    }
-  };
-  auto put = [&](int buf, const DevGemmOp& op, int kc) {  // the chunk (op, kc) fetched last
-    const int krem = min(TK, op.k - kc);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      int r, kk, kb, c;
-      a_at(op, q, r, kk);
-      b_at(op, q, kb, c);
-      As[buf][kk][r] = (r < mrem && kk < krem) ? op.alpha * ra[q] : 0.0;
-      Bs[buf][kb][c] = (c < nrem && kb < krem) ? rb[q] : 0.0;
-    }
-  };
-  int buf = 0;
-  if (o < t.nop) fetch();
-  while (o < t.nop) {
-    const DevGemmOp op = ops[t.op0 + o];
-    put(buf, op, k0);
-    __syncthreads();
-    k0 += TK;
-    skip();
-    if (o < t.nop) fetch();  // in flight while this chunk computes
-#pragma unroll
-    for (int ks = 0; ks < TK / 4; ks++) {  // k past the product's end is zero in LDS
-      const int kk = 4 * ks + lg;
-#pragma unroll
-      for (int q = 0; q < C; q++)
-        acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(As[buf][kk][offa[q]], Bs[buf][kk][offb[q]], acc[q], 0, 0, 0);
-    }
-    buf ^= 1;
-  }
-  double* Cp = tile_out(t, ybase, pbase);
-  const bool add = (t.flags & 2) != 0;
-#pragma unroll
-  for (int q = 0; q < C; q++) {
-    if (!on[q]) continue;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int rr = 16 * si[q] + 4 * r + lg, cc = 16 * sj[q] + lr;
-      if (rr < mrem && cc < nrem) {
-        double* p = Cp + (size_t)(t.m0 + rr) + (size_t)t.ldc * (t.n0 + cc);
-        *p = add ? *p + acc[q][r] : acc[q][r];
-      }
-    }
-  }
-}
-
-// tiles_fit_body for tiles without axpy products (TILE_NO_AXPY): the record of the next
-// product comes in a product ahead as one vector load of a 32-bit word per lane (read with
-// v_readlane when due), so a product switch does not wait for a scalar load before the
-// next chunk's operands can be requested.
-struct FitOp {
-  const double* A;
-  const double* B;
-  double alpha;
-  int lda, ldb, k, ta, tb;
-};
-template <int C>
-__device__ __forceinline__ void tiles_fit_body_pf(const DevTile& t, const DevGemmOp* __restrict__ ops,
-                                                  const double* __restrict__ xbase, double* __restrict__ ybase,
-                                                  double* __restrict__ pbase, double (*As)[TK][TM + 1],
-                                                  double (*Bs)[TK][TN + 1], int ms, int nsub) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, lr = lane & 15, lg = lane >> 4;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int mrem = min(TM, t.m - t.m0), nrem = min(TN, t.n - t.n0);
   int si[C], sj[C], offa[C], offb[C];
   bool on[C];
 #pragma unroll
@@ -432,6 +330,7 @@ __device__ __forceinline__ void tiles_fit_body_pf(const DevTile& t, const DevGem
   chm_t4 acc[C];
 #pragma unroll
   for (int q = 0; q < C; q++) acc[q] = chm_t4{0.0, 0.0, 0.0, 0.0};
+  if (!(t.flags & TILE_NO_AXPY)) tile_axpys<C>(acc, si, sj, on, t, ops, xbase, mrem, nrem, lane);
   const uint32_t* __restrict__ ow = (const uint32_t*)(ops + t.op0);
   auto op_words = [&](int i) -> uint32_t {
     return (i < t.nop && lane < 14) ? ((__attribute__((address_space(1))) const uint32_t*)ow)[(size_t)i * 14 + lane] : 0u;
@@ -453,23 +352,27 @@ __device__ __forceinline__ void tiles_fit_body_pf(const DevTile& t, const DevGem
   auto b_at = [&](const FitOp& op, int q, int& kb, int& c) {
     if (op.tb == 0) { kb = tid & 15; c = (tid >> 4) + 16 * q; } else { c = tid & 63; kb = (tid >> 6) + 4 * q; }
   };
-  double ra[4], rb[4];
-  auto fetch = [&](const FitOp& op, int kc) {  // raw global loads of chunk (op, kc)
-    gdbl* A = (gdbl*)op.A;
-    gdbl* B = (gdbl*)op.B;
+  // raw global (not flat) loads of chunk (op, kc), with 32-bit byte offsets off a uniform base
+  // (a block holds fewer than 2^28 elements); a lane outside the block reads the block's first
+  // element: put applies the masks and alpha, so nothing here waits for the loads
+  auto fetch = [&](const FitOp& op, int kc, double (&ra)[4], double (&rb)[4]) {
+    gbyte* A = (gbyte*)op.A;
+    gbyte* B = (gbyte*)op.B;
     const int krem = min(TK, op.k - kc);
+    const uint32_t a_k = op.ta ? 1u : (uint32_t)op.lda, a_r = op.ta ? (uint32_t)op.lda : 1u;
+    const uint32_t b_k = op.tb ? (uint32_t)op.ldb : 1u, b_c = op.tb ? 1u : (uint32_t)op.ldb;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       int r, kk, kb, c;
       a_at(op, q, r, kk);
       b_at(op, q, kb, c);
-      const size_t ia = op.ta ? (size_t)(kc + kk) + (size_t)op.lda * (t.m0 + r) : (size_t)(t.m0 + r) + (size_t)op.lda * (kc + kk);
-      const size_t ib = op.tb ? (size_t)(t.n0 + c) + (size_t)op.ldb * (kc + kb) : (size_t)(kc + kb) + (size_t)op.ldb * (t.n0 + c);
-      ra[q] = A[(r < mrem && kk < krem) ? ia : 0];
-      rb[q] = B[(c < nrem && kb < krem) ? ib : 0];
+      const uint32_t ia = (uint32_t)(kc + kk) * a_k + (uint32_t)(t.m0 + r) * a_r;
+      const uint32_t ib = (uint32_t)(kc + kb) * b_k + (uint32_t)(t.n0 + c) * b_c;
+      ra[q] = *(gdbl*)(A + ((r < mrem && kk < krem) ? ia * 8u : 0u));
+      rb[q] = *(gdbl*)(B + ((c < nrem && kb < krem) ? ib * 8u : 0u));
     }
   };
-  auto put = [&](int buf, const FitOp& op, int kc) {
+  auto put = [&](int buf, const FitOp& op, int kc, const double (&ra)[4], const double (&rb)[4]) {
     const int krem = min(TK, op.k - kc);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -480,7 +383,8 @@ __device__ __forceinline__ void tiles_fit_body_pf(const DevTile& t, const DevGem
       Bs[buf][kb][c] = (c < nrem && kb < krem) ? rb[q] : 0.0;
     }
   };
-  // the chunk sequence: product o (its fields in cur), chunk k0; vN: words of product o + 1
+  // the chunk sequence: product o (its fields in cur), chunk k0; vN: words of product o + 1;
+  // products without an inner dimension (axpys) are passed over
   int o = 0, k0 = 0;
   FitOp cur = decode(op_words(0));
   uint32_t vN = op_words(1);
@@ -497,9 +401,10 @@ __device__ __forceinline__ void tiles_fit_body_pf(const DevTile& t, const DevGem
   int buf = 0;
   FitOp pc = cur;  // the product of the chunk in ra / rb
   int pk = 0;
-  if (o < t.nop) fetch(cur, k0);
+  double ra[4], rb[4];
+  if (o < t.nop) fetch(cur, k0, ra, rb);
   while (o < t.nop) {
-    put(buf, pc, pk);
+    put(buf, pc, pk, ra, rb);
     __syncthreads();
     k0 += TK;
     if (k0 >= cur.k) {
@@ -507,7 +412,7 @@ __device__ __forceinline__ void tiles_fit_body_pf(const DevTile& t, const DevGem
       next_op();
     }
     if (o < t.nop) {
-      fetch(cur, k0);  // in flight while this chunk computes
+      fetch(cur, k0, ra, rb);  // in flight while this chunk computes
       pc = cur;
       pk = k0;
     }
@@ -544,15 +449,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   const DevTile t = tiles[blockIdx.x];
   const int mrem = min(TM, t.m - t.m0), nrem = min(TN, t.n - t.n0);
   const int ms = (mrem + 15) >> 4, ns = (nrem + 15) >> 4, nsub = ms * ns;
-  if (t.flags & TILE_NO_AXPY) {
-    switch ((nsub + 3) >> 2) {
-      case 1: tiles_fit_body_pf<1>(t, ops, xbase, ybase, pbase, As, Bs, ms, nsub); break;
-      case 2: tiles_fit_body_pf<2>(t, ops, xbase, ybase, pbase, As, Bs, ms, nsub); break;
-      case 3: tiles_fit_body_pf<3>(t, ops, xbase, ybase, pbase, As, Bs, ms, nsub); break;
-      default: tiles_fit_body_pf<4>(t, ops, xbase, ybase, pbase, As, Bs, ms, nsub); break;
-    }
-    return;
-  }
   switch ((nsub + 3) >> 2) {
     case 1: tiles_fit_body<1>(t, ops, xbase, ybase, pbase, As, Bs, ms, nsub); break;
     case 2: tiles_fit_body<2>(t, ops, xbase, ybase, pbase, As, Bs, ms, nsub); break;
@@ -890,9 +786,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 8))) void
   }
 }
 
-// Grouped tiles (DevTile + DevGemmOp lists, phase 2) of at most 32 x 32 whose products are
-// all GEMMs with k > 0: one wavefront per tile walks the chunks of its products; the next
-// product's record comes in a product ahead.
+// Grouped tiles (DevTile + DevGemmOp lists, phase 2 and updates) of at most 16 MS x 16 NS
+// elements: one wavefront per tile adds the tile's axpy products, then walks the chunks of
+// the others; the next product's record comes in a product ahead.
+template <int MS, int NS>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_tiles_wave2(
     const DevTile* __restrict__ tiles, int ntiles, const DevGemmOp* __restrict__ ops, const double* __restrict__ xbase,
     double* __restrict__ ybase, double* __restrict__ pbase) {
@@ -900,18 +797,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 8))) void
   const int ti = blockIdx.x * (NT / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (ti >= ntiles) return;
   const DevTile t = tiles[ti];
-  if (t.nop <= 0) {
-    chm_t4 z[2][2];
-    tw_zero(z);
-    tw_store(z, tile_out(t, ybase, pbase), t.ldc, t.m0, t.n0, min(32, t.m - t.m0), min(32, t.n - t.n0),
-             (t.flags & 2) != 0, lr, lg);
-    return;
-  }
+  const int mrem = min(16 * MS, t.m - t.m0), nrem = min(16 * NS, t.n - t.n0);
   const uint32_t* __restrict__ ow = (const uint32_t*)(ops + t.op0);
   auto op_words = [&](int i) -> uint32_t {
     return (i < t.nop && lane < 14) ? ((__attribute__((address_space(1))) const uint32_t*)ow)[(size_t)i * 14 + lane] : 0u;
   };
-  const int mrem = min(32, t.m - t.m0), nrem = min(32, t.n - t.n0);  // the wavefront's 32 x 32
   auto as_op = [&](uint32_t v) {
     TwOp f;
     const int fl = ts_rl(v, 12);
@@ -924,36 +814,165 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     f.m0 = t.m0; f.n0 = t.n0; f.mrem = mrem; f.nrem = nrem;
     return f;
   };
+  chm_t4 acc[MS][NS];
+  tw_zero(acc);
+  if (!(t.flags & TILE_NO_AXPY)) {
+    chm_t4 flat[MS * NS];
+    int si[MS * NS], sj[MS * NS];
+    bool on[MS * NS];
+#pragma unroll
+    for (int q = 0; q < MS * NS; q++) {
+      flat[q] = chm_t4{0.0, 0.0, 0.0, 0.0};
+      si[q] = q / NS;
+      sj[q] = q % NS;
+      on[q] = true;
+    }
+    tile_axpys<MS * NS>(flat, si, sj, on, t, ops, xbase, mrem, nrem, lane);
+#pragma unroll
+    for (int q = 0; q < MS * NS; q++) acc[q / NS][q % NS] = flat[q];
+  }
   int o = 0, k0 = 0;
   TwOp f = as_op(op_words(0));
   uint32_t vN = op_words(1);
-  chm_t4 acc[2][2];
-  tw_zero(acc);
+  auto next_op = [&]() -> bool {  // to the next product with an inner dimension
+    for (;;) {
+      o++;
+      if (o >= t.nop) return false;
+      f = as_op(vN);
+      vN = op_words(o + 1);
+      if (f.k > 0) return true;
+    }
+  };
   auto advance = [&]() -> bool {
     k0 += TK;
     if (k0 < f.k) return true;
-    o++;
-    if (o >= t.nop) return false;
     k0 = 0;
-    f = as_op(vN);
-    vN = op_words(o + 1);
-    return true;
+    return next_op();
   };
-  double a0[4][2], b0[4][2], a1[4][2], b1[4][2];
-  tw_fetch(f, k0, lr, lg, a0, b0);
-  for (;;) {
-    tw_take(f, k0, lr, lg, a0, b0);
-    bool more = advance();
-    if (more) tw_fetch(f, k0, lr, lg, a1, b1);  // in flight while chunk 0 computes
-    tw_mma(acc, a0, b0);
-    if (!more) break;
-    tw_take(f, k0, lr, lg, a1, b1);
-    more = advance();
-    if (more) tw_fetch(f, k0, lr, lg, a0, b0);
-    tw_mma(acc, a1, b1);
-    if (!more) break;
+  if (t.nop > 0 && (f.k > 0 || next_op())) {
+    double a0[4][MS], b0[4][NS], a1[4][MS], b1[4][NS];
+    tw_fetch(f, k0, lr, lg, a0, b0);
+    for (;;) {
+      tw_take(f, k0, lr, lg, a0, b0);
+      bool more = advance();
+      if (more) tw_fetch(f, k0, lr, lg, a1, b1);  // in flight while chunk 0 computes
+      tw_mma(acc, a0, b0);
+      if (!more) break;
+      tw_take(f, k0, lr, lg, a1, b1);
+      more = advance();
+      if (more) tw_fetch(f, k0, lr, lg, a0, b0);
+      tw_mma(acc, a1, b1);
+      if (!more) break;
+    }
   }
   tw_store(acc, tile_out(t, ybase, pbase), t.ldc, t.m0, t.n0, mrem, nrem, (t.flags & 2) != 0, lr, lg);
+}
+
+// Phase 1 of a long list with the input block in LDS: a workgroup loads its group's columns
+// (or rows) of x once, zero-padded; its wavefronts then walk the group's W, 16 rows (columns)
+// of the operator at a time, without barriers: a strip's operator elements come straight
+// into registers, the next strip's in flight while this one computes. Roles in the MFMA
+// are chosen so that W is stored along its columns. Before, every W was a tile of its own
+// that staged both operands (k_tiles_stream1, k_tiles_wave1): 5.0 ms for the 1.23 M W (42 GF,
+// 4.4 GB written) of the L = 32, D = 2000 middle site, 3.7 ms here.
+static_assert(sizeof(DevStripW) == 32, "DevStripW words");
+template <int NT_, int KC, bool RIGHT>
+__device__ __forceinline__ void strips_body(const DevXGroup& g, const DevStripW* __restrict__ ws,
+                                            const double* __restrict__ x, double* __restrict__ xs) {
+  constexpr int LD = 16 * NT_ + 4;  // 4 (mod 8): the four k rows of a read fall on different banks
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const double* xb = x + g.xoff;
+  for (int e = tid; e < 16 * KC * 16 * NT_; e += NT) {
+    // along the contiguous direction of x
+    const int kk = RIGHT ? e / (16 * NT_) : e % (16 * KC), i = RIGHT ? e % (16 * NT_) : e / (16 * KC);
+    const bool in = kk < g.k && i < g.ni;
+    xs[kk * LD + i] = in ? (RIGHT ? xb[(size_t)(g.i0 + i) + (size_t)g.ld * kk] : xb[(size_t)kk + (size_t)g.ld * (g.i0 + i)]) : 0.0;
+  }
+  __syncthreads();
+  const uint32_t* __restrict__ wwords = (const uint32_t*)(ws + g.w0);
+  auto rec = [&](int i) -> uint32_t {
+    return (i < g.nw && lane < 8) ? ((__attribute__((address_space(1))) const uint32_t*)wwords)[(size_t)i * 8 + lane] : 0u;
+  };
+  struct W {
+    const double* E;
+    double* O;
+    int sj, sk, len, ldc;
+  };
+  auto decode = [&](uint32_t v) {
+    return W{(const double*)ts_rl64(v, 0), (double*)ts_rl64(v, 2), ts_rl(v, 4), ts_rl(v, 5), ts_rl(v, 6), ts_rl(v, 7)};
+  };
+  int wi = wv, j0 = 0;
+  if (wi >= g.nw) return;
+  W f = decode(rec(wi));               // the strip being fetched: rows j0 .. of W f
+  uint32_t vN = rec(wi + NT / 64);
+  auto fetch = [&](double (&o)[4 * KC]) {
+    gbyte* E = (gbyte*)f.E;
+    const uint32_t base = (uint32_t)(j0 + lr) * (uint32_t)f.sj;
+    const bool jok = j0 + lr < f.len;
+#pragma unroll
+    for (int s = 0; s < 4 * KC; s++) {
+      const uint32_t kk = 4 * s + lg;
+      o[s] = *(gdbl*)(E + ((jok && (int)kk < g.k) ? (base + kk * (uint32_t)f.sk) * 8u : 0u));
+    }
+  };
+  auto advance = [&]() -> bool {
+    j0 += 16;
+    if (j0 < f.len) return true;
+    wi += NT / 64;
+    if (wi >= g.nw) return false;
+    j0 = 0;
+    f = decode(vN);
+    vN = rec(wi + NT / 64);
+    return true;
+  };
+  auto compute = [&](const double (&o)[4 * KC], const W& c, int cj) {
+    chm_t4 acc[NT_];
+#pragma unroll
+    for (int t = 0; t < NT_; t++) acc[t] = chm_t4{0.0, 0.0, 0.0, 0.0};
+    const bool jok = cj + lr < c.len;
+#pragma unroll
+    for (int s = 0; s < 4 * KC; s++) {
+      const double ov = (jok && 4 * s + lg < g.k) ? o[s] : 0.0;
+#pragma unroll
+      for (int t = 0; t < NT_; t++) {
+        const double xv = xs[(4 * s + lg) * LD + 16 * t + lr];
+        acc[t] = RIGHT ? __builtin_amdgcn_mfma_f64_16x16x4f64(ov, xv, acc[t], 0, 0, 0)
+                       : __builtin_amdgcn_mfma_f64_16x16x4f64(xv, ov, acc[t], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < NT_; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int i = 16 * t + (RIGHT ? lr : 4 * r + lg), j = cj + (RIGHT ? 4 * r + lg : lr);
+        if (i < g.ni && j < c.len) c.O[RIGHT ? (size_t)(g.i0 + i) + (size_t)c.ldc * j : (size_t)j + (size_t)c.ldc * (g.i0 + i)] = acc[t][r];
+      }
+  };
+  double o0[4 * KC], o1[4 * KC];
+  fetch(o0);
+  for (;;) {
+    W c = f;
+    int cj = j0;
+    bool more = advance();
+    if (more) fetch(o1);  // in flight while this strip computes
+    compute(o0, c, cj);
+    if (!more) break;
+    c = f;
+    cj = j0;
+    more = advance();
+    if (more) fetch(o0);
+    compute(o1, c, cj);
+    if (!more) break;
+  }
+}
+template <int NT_, int KC>
+__global__ __launch_bounds__(NT) void k_strips(const DevXGroup* __restrict__ groups, const DevStripW* __restrict__ ws,
+                                               const double* __restrict__ x) {
+  extern __shared__ double xs[];
+  const DevXGroup g = groups[blockIdx.x];
+  if (g.right) strips_body<NT_, KC, true>(g, ws, x, xs);
+  else strips_body<NT_, KC, false>(g, ws, x, xs);
 }
 
 // Assembles the explicit sub-block of every (kappa, kappa') pair:
@@ -2294,6 +2313,32 @@ void launch_tiles(const DevTile* tiles, const DevGemmOp* ops, int ntiles, const 
   else hipLaunchKernelGGL(k_tiles, dim3(ntiles), dim3(NT), 0, s, tiles, ops, xbase, ybase, pbase);
 }
 
+typedef void (*StripKernel)(const DevXGroup*, const DevStripW*, const double*);
+static constexpr StripKernel STRIP_KERNELS[STRIP_BUCKETS] = {
+    k_strips<1, 1>, k_strips<2, 1>, k_strips<3, 1>, k_strips<4, 1>, k_strips<1, 2>, k_strips<2, 2>, k_strips<3, 2>,
+    k_strips<4, 2>, k_strips<1, 3>, k_strips<2, 3>, k_strips<3, 3>, k_strips<4, 3>, k_strips<1, 4>, k_strips<2, 4>,
+    k_strips<3, 4>, k_strips<4, 4>, k_strips<1, 6>, k_strips<2, 6>, k_strips<3, 6>, k_strips<4, 6>, k_strips<1, 8>,
+    k_strips<2, 8>, k_strips<3, 8>, k_strips<4, 8>};
+static int strip_lds(int bucket) {
+  static constexpr int kc[6] = {1, 2, 3, 4, 6, 8};
+  return 16 * kc[bucket / 4] * (16 * (bucket % 4 + 1) + 4) * (int)sizeof(double);
+}
+
+bool strip_kernel_setup() {
+  bool ok = true;
+  for (int b = 0; b < STRIP_BUCKETS; b++)
+    if (strip_lds(b) > 64 * 1024)
+      ok = hipFuncSetAttribute((const void*)STRIP_KERNELS[b], hipFuncAttributeMaxDynamicSharedMemorySize, strip_lds(b)) ==
+               hipSuccess && ok;
+  return ok;
+}
+
+void launch_strips(const DevXGroup* groups, int ngroups, const DevStripW* ws, int bucket, const double* xbase,
+                   hipStream_t s) {
+  if (ngroups <= 0 || bucket < 0 || bucket >= STRIP_BUCKETS) return;
+  hipLaunchKernelGGL(STRIP_KERNELS[bucket], dim3(ngroups), dim3(NT), strip_lds(bucket), s, groups, ws, xbase);
+}
+
 void launch_tiles_stream1(const DevTile1* tiles, int ntiles, int c, const double* xbase, hipStream_t s) {
   if (ntiles <= 0) return;
   if (c == 0) {  // tiles of at most 32 x 32: one wavefront each
@@ -2316,10 +2361,13 @@ void launch_tiles_stream1(const DevTile1* tiles, int ntiles, int c, const double
   }
 }
 
-void launch_tiles_wave2(const DevTile* tiles, const DevGemmOp* ops, int ntiles, const double* xbase, double* ybase,
-                        hipStream_t s, double* pbase) {
+void launch_tiles_wave2(const DevTile* tiles, const DevGemmOp* ops, int ntiles, int shape, const double* xbase,
+                        double* ybase, hipStream_t s, double* pbase) {
   if (ntiles <= 0) return;
-  hipLaunchKernelGGL(k_tiles_wave2, dim3((ntiles + 3) / 4), dim3(NT), 0, s, tiles, ntiles, ops, xbase, ybase, pbase);
+  typedef void (*Kernel)(const DevTile*, int, const DevGemmOp*, const double*, double*, double*);
+  static constexpr Kernel k[4] = {k_tiles_wave2<1, 1>, k_tiles_wave2<1, 2>, k_tiles_wave2<2, 1>, k_tiles_wave2<2, 2>};
+  hipLaunchKernelGGL(k[shape], dim3((ntiles + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, s, tiles, ntiles, ops, xbase, ybase,
+                     pbase);
 }
 
 void launch_assemble(const DevPair* pairs, const DevKTerm* terms, int64_t npairs, double* M, int64_t nnz, bool split,
