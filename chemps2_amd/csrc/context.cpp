@@ -1444,10 +1444,16 @@ void Ctx::run_terms(const std::vector<UTerm>& terms, const std::vector<std::pair
 // Executes update terms: every output block is overwritten by the sum of its terms.
 // Three-operand terms first form W = alpha op(A) op(B); then every output block sums its
 // two-operand products, W op(C) and the transposed axpys. Products whose blocks are
-// small run in k_ops (2 x 2 register tiles, output blocks with many products split
-// over several work items and summed by k_part_reduce), the rest in k_tiles. The lists
-// are built on the host threads; positions come from prefix sums, so they do not
-// depend on the thread count.
+// small may run in k_ops (2 x 2 register tiles, output blocks with many products split
+// over several work items and summed by k_part_reduce; CHM_OPS_KERNEL). All others are
+// tiles: phase 1 in the kernels of one product per tile that the Heff's intermediates use
+// (a bucket for each shape, the next chunk loaded while this one is multiplied), phase 2 on
+// one wavefront up to 32 x 32 and on a workgroup above. A workgroup for each 64 x 64 tile,
+// whatever its size, was bound by the latency of its few chunks and four wavefronts of
+// which most had no rows: the updates of a sweep at L = 14, D = 250 took 50 ms in it and
+// take 27 ms now, an operator slot at L = 32, D = 2000 (sites 15) 117.9 -> 112.6 ms with
+// its lists. The lists are built on the host threads; positions come from prefix sums, so
+// they do not depend on the thread count.
 void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<Ref, std::pair<int, int>>>& outs,
                     const double* combo_base) {
   const double t_begin = now_s();
@@ -1501,7 +1507,17 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
   };
   const bool ops_on = use_ops_kernel;
   // output block of every term; phase-1 counts per segment (k_ops items or GEMM tiles)
-  struct P1 { int64_t ops = 0, tiles = 0, items = 0, w = 0; };
+  struct P1 {
+    int64_t ops = 0, items = 0, w = 0;
+    std::array<int64_t, TILE_BUCKETS> tiles{};
+  };
+  auto each_tile1 = [](int m, int nn, auto&& f) {  // 64 x 64 tiles by bucket (tile_bucket)
+    for (int m0 = 0; m0 < m; m0 += 64)
+      for (int n0 = 0; n0 < nn; n0 += 64) {
+        const int mr = std::min(64, m - m0), nr = std::min(64, nn - n0);
+        f(m0, n0, mr, nr, tile_bucket(mr, nr));
+      }
+  };
   std::vector<P1> p1(nseg + 1);
   parallel_for(nseg, nthr, [&](int64_t s, int) {
     P1 c;
@@ -1518,15 +1534,19 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
       if (u.kind != 1) continue;
       c.ops++;
       if (ops_on && small_gemm(u.m, u.k2, u.k1, u.ta, u.lda, u.tb, u.ldb)) c.items++;
-      else c.tiles += (int64_t)((u.m + 63) / 64) * ((u.k2 + 63) / 64);
+      else each_tile1(u.m, u.k2, [&](int, int, int, int, int b) { c.tiles[b]++; });
       c.w += ((int64_t)u.m * u.k2 + 7) / 8 * 8;
     }
     p1[s + 1] = c;
   });
   for (int64_t s = 0; s < nseg; s++) {
-    p1[s + 1].ops += p1[s].ops; p1[s + 1].tiles += p1[s].tiles; p1[s + 1].items += p1[s].items; p1[s + 1].w += p1[s].w;
+    p1[s + 1].ops += p1[s].ops; p1[s + 1].items += p1[s].items; p1[s + 1].w += p1[s].w;
+    for (int b = 0; b < TILE_BUCKETS; b++) p1[s + 1].tiles[b] += p1[s].tiles[b];
   }
-  const int64_t n1 = p1[nseg].ops, nt1 = p1[nseg].tiles, ni1 = p1[nseg].items;
+  // phase-1 tiles bucket after bucket: bucket b at [b1[b], b1[b + 1])
+  std::array<int64_t, TILE_BUCKETS + 1> b1{};
+  for (int b = 0; b < TILE_BUCKETS; b++) b1[b + 1] = b1[b] + p1[nseg].tiles[b];
+  const int64_t n1 = p1[nseg].ops, nt1 = b1[TILE_BUCKETS], ni1 = p1[nseg].items;
   u_W.alloc(std::max<int64_t>(p1[nseg].w, 1));
   double* Wp = u_W.p;
   // terms grouped by output block, stable in (segment, term) order: a counting sort
@@ -1572,7 +1592,8 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
   const double t_sort = now_s();
   // phase 2 per output block: small path or tiles; counts, then positions
   std::vector<char> qsmall(nq, 0);
-  std::vector<int64_t> t2start(nq + 1, 0), i2start(nq + 1, 0), p2start(nq + 1, 0);
+  // (tiles of at most 32 x 32, one wavefront each, then the rest)
+  std::vector<int64_t> tw2start(nq + 1, 0), t2start(nq + 1, 0), i2start(nq + 1, 0), p2start(nq + 1, 0);
   parallel_for((nq + 1023) / 1024, nthr, [&](int64_t c, int) {
     for (int64_t q = c * 1024; q < std::min<int64_t>(nq, (c + 1) * 1024); q++) {
       const int m = outs[q].second.first, nn = outs[q].second.second;
@@ -1591,24 +1612,25 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
         i2start[q + 1] = ni;
         p2start[q + 1] = ni > 1 ? ni * (int64_t)m * nn : 0;
       } else {
-        t2start[q + 1] = (int64_t)((m + 63) / 64) * ((nn + 63) / 64);
+        each_tile1(m, nn, [&](int, int, int mr, int nr, int) { (mr <= 32 && nr <= 32 ? tw2start : t2start)[q + 1]++; });
       }
     }
   });
   int64_t nred = 0;
   for (int64_t q = 0; q < nq; q++) {
     if (qsmall[q] && i2start[q + 1] > 1) nred++;
-    t2start[q + 1] += t2start[q]; i2start[q + 1] += i2start[q]; p2start[q + 1] += p2start[q];
+    tw2start[q + 1] += tw2start[q]; t2start[q + 1] += t2start[q]; i2start[q + 1] += i2start[q]; p2start[q + 1] += p2start[q];
   }
-  const int64_t nt2 = t2start[nq], ni2 = i2start[nq], npart = p2start[nq];
+  const int64_t ntw2 = tw2start[nq], nt2 = ntw2 + t2start[nq], ni2 = i2start[nq], npart = p2start[nq];
   if (nt1 > INT32_MAX || nt2 > INT32_MAX || ni1 + ni2 > INT32_MAX) throw Error{ERR_SIZE, "too many update tiles"};
   const double t_counts = now_s();
   ustage.reset();
-  ustage.reserve(256 * 8 + (n1 + n) * sizeof(DevGemmOp) + (nt1 + nt2) * sizeof(DevTile) + (ni1 + ni2) * sizeof(DevOItem) +
-                 nred * sizeof(DevPRed));
-  DevGemmOp* o1 = ustage.take<DevGemmOp>(n1);
+  const int64_t no1 = ops_on ? n1 : 0;  // phase-1 product records: k_ops only, a tile holds its own
+  ustage.reserve(256 * 8 + (no1 + n) * sizeof(DevGemmOp) + nt1 * sizeof(DevTile1) + nt2 * sizeof(DevTile) +
+                 (ni1 + ni2) * sizeof(DevOItem) + nred * sizeof(DevPRed));
+  DevGemmOp* o1 = ustage.take<DevGemmOp>(no1);
   DevGemmOp* o2 = ustage.take<DevGemmOp>(n);
-  DevTile* t1 = ustage.take<DevTile>(nt1);
+  DevTile1* t1 = ustage.take<DevTile1>(nt1);
   DevTile* t2 = ustage.take<DevTile>(nt2);
   DevOItem* it1 = ustage.take<DevOItem>(ni1);
   DevOItem* it2 = ustage.take<DevOItem>(ni2);
@@ -1621,7 +1643,9 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
   };
   // phase 1: W = alpha op(A) op(B) for three-operand terms
   parallel_for(nseg, nthr, [&](int64_t s, int) {
-    int64_t io = p1[s].ops, it = p1[s].tiles, ii = p1[s].items, iw = p1[s].w;
+    int64_t io = p1[s].ops, ii = p1[s].items, iw = p1[s].w;
+    std::array<int64_t, TILE_BUCKETS> it = p1[s].tiles;
+    for (int b = 0; b < TILE_BUCKETS; b++) it[b] += b1[b];
     const double* cb = combo_base ? combo_base + segs[s].combo_base : nullptr;
     int pl = 1;
     for (size_t j = 0; j < segs[s].terms.size(); j++) {
@@ -1632,19 +1656,20 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
       op.B = resolve_with(u.B, cb); op.tb = u.tb; op.ldb = u.ldb;
       op.k = u.k1; op.alpha = u.alpha; op.kind = 0;
       woff[s0[s] + j] = iw;
-      const int opi = (int)io;
-      o1[io++] = op;
+      if (ops_on) o1[io] = op;
+      const int opi = (int)io++;
       if (ops_on && small_gemm(u.m, u.k2, u.k1, u.ta, u.lda, u.tb, u.ldb)) {
         it1[ii++] = DevOItem{Wp + iw, u.m, u.k2, opi, 1};
         pl = std::max({pl, u.m * u.k1, u.k1 * u.k2});
       } else {
-        for (int m0 = 0; m0 < u.m; m0 += 64)
-          for (int n0 = 0; n0 < u.k2; n0 += 64) {
-            DevTile tl{};
-            tl.C = Wp + iw;
-            tl.ldc = u.m; tl.m0 = m0; tl.n0 = n0; tl.m = u.m; tl.n = u.k2; tl.op0 = opi; tl.nop = 1; tl.flags = TILE_NO_AXPY;
-            t1[it++] = tl;
-          }
+        if (u.k1 <= 0) throw Error{ERR_STATE, "operator update: a product with no inner dimension"};
+        each_tile1(u.m, u.k2, [&](int m0, int n0, int mr, int nr, int b) {
+          DevTile1 tl{};
+          tl.C = Wp + iw; tl.A = op.A; tl.B = op.B; tl.alpha = op.alpha;
+          tl.ldc = u.m; tl.m0 = m0; tl.n0 = n0; tl.mrem = mr; tl.nrem = nr;
+          tl.lda = op.lda; tl.ldb = op.ldb; tl.k = op.k; tl.ta = op.ta; tl.tb = op.tb;
+          t1[it[b]++] = tl;
+        });
       }
       iw += ((int64_t)u.m * u.k2 + 7) / 8 * 8;
     }
@@ -1697,41 +1722,42 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
         for (int64_t pos = qstart[q]; pos < qstart[q + 1]; pos++)
           if (o2[pos].kind == 0) pl = std::max({pl, m * o2[pos].k, o2[pos].k * nn});
       } else {
-        int64_t it = t2start[q];
+        int64_t itw = tw2start[q], it = ntw2 + t2start[q];
         bool axpy = false;
         for (int64_t pos = qstart[q]; pos < qstart[q + 1]; pos++) axpy |= o2[pos].kind == 1;
-        for (int m0 = 0; m0 < m; m0 += 64)
-          for (int n0 = 0; n0 < nn; n0 += 64) {
-            DevTile tl{};
-            tl.C = C; tl.ldc = m; tl.m0 = m0; tl.n0 = n0; tl.m = m; tl.n = nn;
-            tl.op0 = (int)qstart[q]; tl.nop = (int)(qstart[q + 1] - qstart[q]);
-            tl.flags = axpy ? 0 : TILE_NO_AXPY;
-            t2[it++] = tl;
-          }
+        each_tile1(m, nn, [&](int m0, int n0, int mr, int nr, int) {
+          DevTile tl{};
+          tl.C = C; tl.ldc = m; tl.m0 = m0; tl.n0 = n0; tl.m = m; tl.n = nn;
+          tl.op0 = (int)qstart[q]; tl.nop = (int)(qstart[q + 1] - qstart[q]);
+          tl.flags = axpy ? 0 : TILE_NO_AXPY;
+          t2[mr <= 32 && nr <= 32 ? itw++ : it++] = tl;
+        });
       }
     }
     need(pl);
   });
   const double t_lists = now_s();
-  u_d1.alloc(std::max<int64_t>(n1, 1));
+  u_d1.alloc(std::max<int64_t>(no1, 1));
   u_d2.alloc(std::max<int64_t>(n, 1));
   u_dt1.alloc(std::max<int64_t>(nt1, 1));
   u_dt2.alloc(std::max<int64_t>(nt2, 1));
   u_it1.alloc(std::max<int64_t>(ni1, 1));
   u_it2.alloc(std::max<int64_t>(ni2, 1));
   u_rd.alloc(std::max<int64_t>(nred, 1));
-  if (n1) hip_check(hipMemcpyAsync(u_d1.p, o1, n1 * sizeof(DevGemmOp), hipMemcpyHostToDevice, stream), "ops");
+  if (no1) hip_check(hipMemcpyAsync(u_d1.p, o1, no1 * sizeof(DevGemmOp), hipMemcpyHostToDevice, stream), "ops");
   if (n) hip_check(hipMemcpyAsync(u_d2.p, o2, n * sizeof(DevGemmOp), hipMemcpyHostToDevice, stream), "ops");
-  if (nt1) hip_check(hipMemcpyAsync(u_dt1.p, t1, nt1 * sizeof(DevTile), hipMemcpyHostToDevice, stream), "tiles");
+  if (nt1) hip_check(hipMemcpyAsync(u_dt1.p, t1, nt1 * sizeof(DevTile1), hipMemcpyHostToDevice, stream), "tiles");
   if (nt2) hip_check(hipMemcpyAsync(u_dt2.p, t2, nt2 * sizeof(DevTile), hipMemcpyHostToDevice, stream), "tiles");
   if (ni1) hip_check(hipMemcpyAsync(u_it1.p, it1, ni1 * sizeof(DevOItem), hipMemcpyHostToDevice, stream), "items");
   if (ni2) hip_check(hipMemcpyAsync(u_it2.p, it2, ni2 * sizeof(DevOItem), hipMemcpyHostToDevice, stream), "items");
   if (nred) hip_check(hipMemcpyAsync(u_rd.p, rd, nred * sizeof(DevPRed), hipMemcpyHostToDevice, stream), "reductions");
   const double t_up = now_s();
   const int P = std::min(OPS_P, (Pneed.load() + 31) / 32 * 32);
-  launch_tiles(u_dt1.p, u_d1.p, (int)nt1, nullptr, nullptr, stream, tiles_kernel);
+  for (int b = 0; b < TILE_BUCKETS; b++)
+    launch_tiles_stream1(u_dt1.p + b1[b], (int)(b1[b + 1] - b1[b]), b, nullptr, stream);
   launch_ops(u_it1.p, (int)ni1, u_d1.p, P, stream);
-  launch_tiles(u_dt2.p, u_d2.p, (int)nt2, nullptr, nullptr, stream, tiles_kernel);
+  launch_tiles_wave2(u_dt2.p, u_d2.p, (int)ntw2, 3, nullptr, nullptr, stream);
+  launch_tiles(u_dt2.p + ntw2, u_d2.p, (int)(nt2 - ntw2), nullptr, nullptr, stream, tiles_kernel);
   launch_ops(u_it2.p, (int)ni2, u_d2.p, P, stream);
   launch_part_reduce(u_rd.p, (int)nred, u_part.p, stream);
   hip_check(hipGetLastError(), "update kernels");

@@ -297,7 +297,8 @@ struct Ctx : HostState {
   std::vector<int> u_qof, u_seg;
   std::vector<int64_t> u_woff, u_order, u_hist;
   DBuf<DevGemmOp> u_d1, u_d2;
-  DBuf<DevTile> u_dt1, u_dt2;
+  DBuf<DevTile1> u_dt1;
+  DBuf<DevTile> u_dt2;
   DBuf<double> u_W;
   DBuf<DevOItem> u_it1, u_it2;
   DBuf<DevPRed> u_rd;
