@@ -121,6 +121,7 @@ struct OpT {
   int index = 0;  // == boundary (the reference's TensorOperator::gIndex)
   bool moving_right = true, prime_last = true, jw_phase = false;
   int32_t buf = -1;  // buffer id of its device copy
+  bool in_arena = false;  // the copy lies in its set's arena
   int64_t size = 0;
   std::shared_ptr<const SecIndex> bi;  // sector index of the boundary it was laid out on
   std::vector<int64_t> offs;           // [up position * (two_j + 1) + (s' - s + two_j) / 2] -> offset or -1
@@ -156,6 +157,8 @@ struct OpSet {
   std::vector<std::vector<OpT*>> F0, F1, S0, S1, A, B, C, D;
   OpT* X = nullptr;
   std::vector<std::unique_ptr<OpT>> owned;
+  double* arena = nullptr;  // device memory of the tensors laid out together
+  size_t arena_n = 0;       // its doubles
 };
 
 // Two-site object layout (Sobject.cpp:36-147): blocks (NL, 2SL, IL, N1, N2, 2J, NR,

@@ -29,6 +29,8 @@ Ctx::~Ctx() {
   for (auto st : svd_streams)
     if (st) (void)hipStreamDestroy(st);
   if (s_buf >= 0) bufs[s_buf] = nullptr;  // owned by Sdev
+  for (int c = 0; c < (int)sets.size(); c++) clear_set(c);
+  arenas_release();
   for (double* p : bufs)
     if (p) (void)hipFree(p);
   for (auto& e : ev)
@@ -54,6 +56,8 @@ void Ctx::set_problem(int L_, int group_, const int* irr, int N_, int TwoS_, int
   sec.resize(L);
   fci.clear();
   if (s_buf >= 0) bufs[s_buf] = nullptr;  // owned by Sdev
+  for (int c = 0; c < (int)sets.size(); c++) clear_set(c);
+  arenas_release();
   for (double* p : bufs)
     if (p) (void)hipFree(p);
   bufs.assign(BUF_TENSOR0, nullptr);
@@ -91,6 +95,80 @@ void Ctx::set_sectors(int b, int n, const int* Ns, const int* Ss, const int* Is,
   site = -1;
 }
 
+int32_t Ctx::new_buf(double* p, int64_t n) {
+  bufs.push_back(p);
+  buf_len.push_back(n);
+  return (int32_t)bufs.size() - 1;
+}
+
+// n doubles of device memory: a kept arena of at most twice the size, else a new one, where
+// small with some room so that it also serves a slot a little larger.
+double* Ctx::arena_get(size_t n, size_t& cap) {
+  int best = -1;
+  for (int q = 0; q < (int)free_arenas.size(); q++)
+    if (free_arenas[q].second >= n && free_arenas[q].second <= 2 * n + (1 << 16) &&
+        (best < 0 || free_arenas[q].second < free_arenas[best].second))
+      best = q;
+  if (best >= 0) {
+    double* p = free_arenas[best].first;
+    cap = free_arenas[best].second;
+    free_arenas.erase(free_arenas.begin() + best);
+    return p;
+  }
+  double* p = nullptr;
+  cap = n + n / 8 <= ARENA_KEEP ? n + n / 8 : n;
+  if (hipMalloc((void**)&p, cap * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();
+    arenas_release();
+    cap = n;
+    hip_check(hipMalloc((void**)&p, cap * sizeof(double)), "hipMalloc operators");
+  }
+  return p;
+}
+
+void Ctx::arena_put(double* p, size_t cap) {
+  if (cap > ARENA_KEEP) {
+    (void)hipFree(p);
+    return;
+  }
+  (void)hipDeviceSynchronize();  // as a hipFree would: nothing in flight uses the memory still
+  free_arenas.push_back({p, cap});
+  if ((int)free_arenas.size() > FREE_ARENAS) {  // the oldest goes
+    (void)hipFree(free_arenas.front().first);
+    free_arenas.erase(free_arenas.begin());
+  }
+}
+
+void Ctx::arenas_release() {
+  for (auto& a : free_arenas) (void)hipFree(a.first);
+  free_arenas.clear();
+}
+
+OpT** Ctx::tensor_place(OpSet& s, int kind, int k, int m) {
+  auto slot1 = [&](std::vector<OpT*>& v) -> OpT** {
+    if ((int)v.size() <= k) v.resize(k + 1, nullptr);
+    return &v[k];
+  };
+  auto slot2 = [&](std::vector<std::vector<OpT*>>& v) -> OpT** {
+    if ((int)v.size() <= k) v.resize(k + 1);
+    if ((int)v[k].size() <= m) v[k].resize(m + 1, nullptr);
+    return &v[k][m];
+  };
+  switch (kind) {
+    case KIND_L: return slot1(s.L);
+    case KIND_Q: return slot1(s.Q);
+    case KIND_X: return &s.X;
+    case KIND_F0: return slot2(s.F0);
+    case KIND_F1: return slot2(s.F1);
+    case KIND_S0: return slot2(s.S0);
+    case KIND_S1: return slot2(s.S1);
+    case KIND_A: return slot2(s.A);
+    case KIND_B: return slot2(s.B);
+    case KIND_C: return slot2(s.C);
+    default: return slot2(s.D);
+  }
+}
+
 OpT* Ctx::add_tensor(int cnt, bool mr, int kind, int k, int m, int two_j, int n_elec, int n_irrep, int64_t n) {
   if (!have_problem) throw Error{ERR_STATE, "set the problem first"};
   if (cnt < 0 || cnt > L - 2) throw Error{ERR_ARG, "slot out of range"};
@@ -104,55 +182,60 @@ OpT* Ctx::add_tensor(int cnt, bool mr, int kind, int k, int m, int two_j, int n_
   if (n >= 0 && owned->size != n)
     throw Error{ERR_SIZE, "tensor size " + std::to_string(n) + " != layout size " + std::to_string(owned->size)};
   OpT* t = owned.get();
-  auto slot1 = [&](std::vector<OpT*>& v) -> OpT*& {
-    if ((int)v.size() <= k) v.resize(k + 1, nullptr);
-    return v[k];
-  };
-  auto slot2 = [&](std::vector<std::vector<OpT*>>& v) -> OpT*& {
-    if ((int)v.size() <= k) v.resize(k + 1);
-    if ((int)v[k].size() <= m) v[k].resize(m + 1, nullptr);
-    return v[k][m];
-  };
-  OpT** where = nullptr;
-  switch (kind) {
-    case KIND_L: where = &slot1(s.L); break;
-    case KIND_Q: where = &slot1(s.Q); break;
-    case KIND_X: where = &s.X; break;
-    case KIND_F0: where = &slot2(s.F0); break;
-    case KIND_F1: where = &slot2(s.F1); break;
-    case KIND_S0: where = &slot2(s.S0); break;
-    case KIND_S1: where = &slot2(s.S1); break;
-    case KIND_A: where = &slot2(s.A); break;
-    case KIND_B: where = &slot2(s.B); break;
-    case KIND_C: where = &slot2(s.C); break;
-    case KIND_D: where = &slot2(s.D); break;
-  }
-  if (*where) {  // replace: free the old device copy
-    if ((*where)->buf >= 0 && bufs[(*where)->buf]) {
-      (void)hipFree(bufs[(*where)->buf]);
-      bufs[(*where)->buf] = nullptr;
-      buf_len[(*where)->buf] = 0;
-    }
+  OpT** where = tensor_place(s, kind, k, m);
+  if (*where && (*where)->buf >= 0 && bufs[(*where)->buf]) {  // replace: free the old device copy
+    if (!(*where)->in_arena) (void)hipFree(bufs[(*where)->buf]);
+    bufs[(*where)->buf] = nullptr;
+    buf_len[(*where)->buf] = 0;
   }
   double* p = nullptr;
   if (t->size > 0) hip_check(hipMalloc((void**)&p, t->size * sizeof(double)), "hipMalloc tensor");
-  t->buf = (int32_t)bufs.size();
-  bufs.push_back(p);
-  buf_len.push_back(t->size);
+  t->buf = new_buf(p, t->size);
   *where = t;
   s.owned.push_back(std::move(owned));
   site = -1;
   return t;
 }
 
+// Slot cnt emptied and every operator of DMRG::allocateTensors laid out in it (current sectors),
+// in one allocation, each tensor on a 512-byte boundary.
+void Ctx::place_set(int cnt, bool mr) {
+  clear_set(cnt);
+  const std::vector<OpShape> shapes = opset_shapes(*this, cnt, mr);
+  const int64_t n = (int64_t)shapes.size();
+  std::vector<std::unique_ptr<OpT>> ts(n);
+  parallel_for((n + 15) / 16, host_threads(), [&](int64_t c, int) {
+    for (int64_t q = 16 * c; q < std::min(n, 16 * (c + 1)); q++) {
+      ts[q] = std::make_unique<OpT>();
+      ts[q]->build(sec, cnt + 1, shapes[q].two_j, shapes[q].n_elec, shapes[q].n_irrep);
+      ts[q]->in_arena = true;
+    }
+  });
+  size_t total = 0;
+  for (auto& t : ts) total += ((size_t)t->size + 63) / 64 * 64;
+  OpSet& s = sets[cnt];
+  if (total > 0) s.arena = arena_get(total, s.arena_n);
+  s.dir = mr ? 1 : 2;
+  size_t off = 0;
+  for (int64_t q = 0; q < n; q++) {
+    OpT* t = ts[q].get();
+    t->buf = new_buf(t->size > 0 ? s.arena + off : nullptr, t->size);
+    off += ((size_t)t->size + 63) / 64 * 64;
+    *tensor_place(s, shapes[q].kind, shapes[q].k, shapes[q].m) = t;
+    s.owned.push_back(std::move(ts[q]));
+  }
+  site = -1;
+}
+
 void Ctx::clear_set(int cnt) {
   OpSet& s = sets[cnt];
   for (auto& o : s.owned)
     if (o->buf >= 0 && bufs[o->buf]) {
-      (void)hipFree(bufs[o->buf]);
+      if (!o->in_arena) (void)hipFree(bufs[o->buf]);
       bufs[o->buf] = nullptr;
       buf_len[o->buf] = 0;
     }
+  if (s.arena) arena_put(s.arena, s.arena_n);
   s = OpSet();
   site = -1;
 }
@@ -205,9 +288,9 @@ void Ctx::drop_plan() {
 // DMRG::allocateTensors, before their values are computed.
 void Ctx::alloc_slot(int index, bool mr) {
   const int prepared = site;  // a prepared Heff reads slots site - 1 and site + 1 only
-  clear_set(index);
+  place_set(index, mr);
   for (const OpShape& sh : opset_shapes(*this, index, mr)) {
-    OpT* t = add_tensor(index, mr, sh.kind, sh.k, sh.m, sh.two_j, sh.n_elec, sh.n_irrep, -1);
+    OpT* t = *tensor_place(sets[index], sh.kind, sh.k, sh.m);
     t->moving_right = mr;
     t->jw_phase = (sh.kind == KIND_L || sh.kind == KIND_Q);
     t->prime_last = (sh.kind == KIND_F1 || sh.kind == KIND_D) ? mr : true;
@@ -2642,10 +2725,10 @@ int chm_tensor_fill_synthetic(chm_ctx* ctx, int cnt, int moving_right, uint64_t 
   return guard(ctx, [&](Ctx& c) {
     (void)hipSetDevice(c.device);
     if (cnt < 0 || cnt > c.L - 2) throw Error{CHM_ERR_ARG, "slot out of range"};
-    c.clear_set(cnt);
+    c.place_set(cnt, moving_right != 0);
     uint64_t s = seed * 1000003ULL + 17;
     for (const chm::OpShape& sh : chm::opset_shapes(c, cnt, moving_right != 0)) {
-      chm::OpT* t = c.add_tensor(cnt, moving_right != 0, sh.kind, sh.k, sh.m, sh.two_j, sh.n_elec, sh.n_irrep, -1);
+      const chm::OpT* t = *c.tensor_place(c.sets[cnt], sh.kind, sh.k, sh.m);
       const uint64_t ts = s++;  // one seed per tensor in allocation order, empty ones included
       if (t->size > 0) chm::launch_fill_hash(c.bufs[t->buf], t->size, ts, 1.0 / std::sqrt((double)t->size), c.stream);
     }

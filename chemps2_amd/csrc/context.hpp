@@ -8,6 +8,7 @@
 #include "dbuf.hpp"
 #include "heff_plan.hpp"
 #include "learned.hpp"
+#include "parallel.hpp"
 #include "update_plan.hpp"
 
 namespace chm {
@@ -100,6 +101,7 @@ struct LowerState {
 };
 
 struct Ctx : HostState {
+  Pool::Ref pool;  // first, so that it is the last to go: the loops' worker threads
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
@@ -395,6 +397,19 @@ struct Ctx : HostState {
   void set_problem(int L, int group, const int* irr, int N, int TwoS, int Irrep, const double* mx, double econst);
   const double* resolve_with(const Ref& r, const double* combo_base) const;
   void set_sectors(int b, int n, const int* Ns, const int* Ss, const int* Is, const int* ds);
+  // The operators of a slot that are laid out together live in one allocation (a slot has up
+  // to a thousand tensors: as many hipMalloc and hipFree calls for every step of a sweep, each
+  // of some microseconds). Of the small ones given up the last FREE_ARENAS are kept for the
+  // slots that follow; a large one is one call among much work.
+  static constexpr int FREE_ARENAS = 2;
+  static constexpr size_t ARENA_KEEP = 32 << 20;  // doubles
+  std::vector<std::pair<double*, size_t>> free_arenas;
+  double* arena_get(size_t n, size_t& cap);
+  void arena_put(double* p, size_t cap);
+  void arenas_release();
+  int32_t new_buf(double* p, int64_t n);
+  void place_set(int cnt, bool mr);
+  OpT** tensor_place(OpSet& s, int kind, int k, int m);
   OpT* add_tensor(int cnt, bool mr, int kind, int k, int m, int two_j, int n_elec, int n_irrep, int64_t n);
   void clear_set(int cnt);
   void prepare(int site);
@@ -412,6 +427,7 @@ struct Ctx : HostState {
     W.release();
     u_arena.release();
     sw.release();
+    arenas_release();
     M_nnz = 0;
     site = -1;
   }
