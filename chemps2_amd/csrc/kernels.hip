@@ -981,31 +981,87 @@ __global__ __launch_bounds__(NT) void k_strips(const DevXGroup* __restrict__ gro
 // buffer and lo = fl32(v - hi) in the next nnz: hi alone is v to 2^-24, hi + lo (exact
 // in double) is v to 2^-48, in the same bytes as the double matrix.
 template <bool SPLIT>
+__device__ __forceinline__ void assemble_store(double* M, int64_t nnz, int64_t e, double v) {
+  if constexpr (SPLIT) {
+    float* hi = reinterpret_cast<float*>(M);
+    const float h = (float)v;
+    hi[e] = h;
+    hi[nnz + e] = (float)(v - (double)h);
+  } else {
+    M[e] = v;
+  }
+}
+// A thread takes one (l, l') and J of the (r, r'): alpha a is one load and one product for J
+// elements, and an element and term costs one load, one multiply-add and its address. With
+// an element a thread the kernel was bound by two dependent loads and some 25 instructions of
+// address work per term. J = 8 from 2048 elements on, where every thread still has work, 2
+// from 512; U terms are in flight where J is small. Each element's sum keeps its order.
+// Before and now: L = 24, D = 1000 site 5.6 -> 3.4 ms, L = 32, D = 2000 8.8 -> 5.0 ms,
+// Hubbard L = 12, D = 200 241 -> 83 us; many small blocks (L = 14, D = 250) 65 -> 80 us, for
+// 76 registers a thread leave six instead of eight wavefronts to hide latency (64 registers
+// by spilling: 61 us there, but 5.2 and 7.7 ms in the first two).
+template <bool SPLIT, int J>
+__device__ __forceinline__ void assemble_body(const DevPair& p, const DevKTerm* __restrict__ terms, double* __restrict__ M,
+                                              int64_t nnz) {
+  const int dR = p.R / p.dL, nf = dR * p.dRi, na = p.dL * p.dLi;
+  const int n = na * ((nf + J - 1) / J);
+  for (int u = threadIdx.x; u < n; u += 256) {
+    const int c = u / na, w = u - c * na;
+    const int li = w / p.dL, l = w - li * p.dL;
+    int r[J], ri[J];
+    ri[0] = c * J / dR;
+    r[0] = c * J - ri[0] * dR;
+#pragma unroll
+    for (int j = 1; j < J; j++) {
+      const bool wrap = r[j - 1] + 1 == dR;
+      r[j] = wrap ? 0 : r[j - 1] + 1;
+      ri[j] = ri[j - 1] + (wrap ? 1 : 0);
+    }
+    double v[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) v[j] = 0.0;
+    auto fetch = [&](int q, double& a, double (&b)[J]) {
+      const DevKTerm t = terms[p.t0 + q];
+      a = t.alpha * (t.A ? (t.ta ? t.A[li + (size_t)t.lda * l] : t.A[l + (size_t)t.lda * li]) : (l == li ? 1.0 : 0.0));
+      if (t.B) {
+        const unsigned s1 = t.tb ? 1 : t.ldb, s2 = t.tb ? t.ldb : 1;
+#pragma unroll
+        for (int j = 0; j < J; j++) b[j] = t.B[ri[j] < p.dRi ? (unsigned)r[j] * s1 + (unsigned)ri[j] * s2 : 0u];
+      } else {
+#pragma unroll
+        for (int j = 0; j < J; j++) b[j] = r[j] == ri[j] ? 1.0 : 0.0;
+      }
+    };
+    constexpr int U = J >= 8 ? 1 : J >= 2 ? 2 : 4;
+    int q = 0;
+    for (; q + U <= p.nt; q += U) {
+      double a[U], b[U][J];
+#pragma unroll
+      for (int w2 = 0; w2 < U; w2++) fetch(q + w2, a[w2], b[w2]);
+#pragma unroll
+      for (int w2 = 0; w2 < U; w2++)
+#pragma unroll
+        for (int j = 0; j < J; j++) v[j] = fma(a[w2], b[w2][j], v[j]);
+    }
+    for (; U > 1 && q < p.nt; q++) {
+      double a, b[J];
+      fetch(q, a, b);
+#pragma unroll
+      for (int j = 0; j < J; j++) v[j] = fma(a, b[j], v[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < J; j++)
+      if (ri[j] < p.dRi) assemble_store<SPLIT>(M, nnz, p.moff + (l + (int64_t)p.dL * r[j]) + (int64_t)p.R * (li + p.dLi * ri[j]), v[j]);
+  }
+}
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_assemble(const DevPair* __restrict__ pairs, const DevKTerm* __restrict__ terms,
                                                   double* __restrict__ M, int64_t nnz) {
   const DevPair p = pairs[blockIdx.x];
-  const int ncol = p.dLi * p.dRi;
-  const int n = p.R * ncol;
-  for (int e = threadIdx.x; e < n; e += 256) {
-    const int row = e % p.R, col = e / p.R;
-    const int l = row % p.dL, r = row / p.dL;
-    const int li = col % p.dLi, ri = col / p.dLi;
-    double v = 0.0;
-    for (int q = 0; q < p.nt; q++) {
-      const DevKTerm t = terms[p.t0 + q];
-      const double a = t.A ? (t.ta ? t.A[li + (size_t)t.lda * l] : t.A[l + (size_t)t.lda * li]) : (l == li ? 1.0 : 0.0);
-      const double b = t.B ? (t.tb ? t.B[r + (size_t)t.ldb * ri] : t.B[ri + (size_t)t.ldb * r]) : (r == ri ? 1.0 : 0.0);
-      v += t.alpha * a * b;
-    }
-    if constexpr (SPLIT) {
-      float* hi = reinterpret_cast<float*>(M);
-      const float h = (float)v;
-      hi[p.moff + e] = h;
-      hi[nnz + p.moff + e] = (float)(v - (double)h);
-    } else {
-      M[p.moff + e] = v;
-    }
-  }
+  const int n = p.R * p.dLi * p.dRi;
+  if (n >= 8 * 256) assemble_body<SPLIT, 8>(p, terms, M, nnz);
+  else if (n >= 2 * 256) assemble_body<SPLIT, 2>(p, terms, M, nnz);
+  else assemble_body<SPLIT, 1>(p, terms, M, nnz);
 }
 
 // Explicit block product, pass 1: one workgroup per work item (at most BX_COLS
