@@ -1533,10 +1533,10 @@ void Ctx::run_terms(const std::vector<UTerm>& terms, const std::vector<std::pair
 // (a bucket for each shape, the next chunk loaded while this one is multiplied), phase 2 on
 // one wavefront up to 32 x 32 and on a workgroup above. A workgroup for each 64 x 64 tile,
 // whatever its size, was bound by the latency of its few chunks and four wavefronts of
-// which most had no rows: the updates of a sweep at L = 14, D = 250 took 50 ms in it and
-// take 27 ms now, an operator slot at L = 32, D = 2000 (sites 15) 117.9 -> 112.6 ms with
-// its lists. The lists are built on the host threads; positions come from prefix sums, so
-// they do not depend on the thread count.
+// which most had no rows: the tiles of a whole solve at L = 14, D = 250 took 25 ms in it
+// and take 14 ms now; an operator move with the lists and product of the next site at
+// L = 32, D = 2000 117.9 -> 112.6 ms. The lists are built on the host threads; positions
+// come from prefix sums, so they do not depend on the thread count.
 void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<Ref, std::pair<int, int>>>& outs,
                     const double* combo_base) {
   const double t_begin = now_s();
