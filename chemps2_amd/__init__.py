@@ -28,6 +28,7 @@ EXPORTS = [
     "chm_mlp_train", "chm_harvest", "chm_harvest_take", "chm_dmrg_sweep_range",
     "chm_dmrg_new_excitation", "chm_dmrg_nstates", "chm_dmrg_site_log", "chm_dmrg_2rdm", "chm_heff_apply_noalloc", "chm_davidson_stats",
     "chm_set_heff_knobs", "chm_set_tuning", "chm_tuning_used", "chm_precond_stats",
+    "chm_split_stats",
 ]
 PRECOND_DIAGONAL, PRECOND_LEARNED = 0, 1
 MLP_IN, MLP_H = 8, 128
@@ -76,6 +77,7 @@ def load():
         "chm_dmrg_2rdm": (i, [vp, C.c_void_p, C.c_void_p, C.POINTER(C.c_double)]),
         "chm_heff_apply_noalloc": (i, [vp, C.c_void_p, C.c_void_p]),
         "chm_davidson_stats": (i, [vp, C.POINTER(C.c_int64)]),
+        "chm_split_stats": (i, [vp, C.POINTER(C.c_int64)]),
         "chm_dmrg_site_log": (i, [vp, C.POINTER(i), vp, vp, vp]),
         "chm_set_heff_knobs": (i, [vp, i64, i, i, i, i]),
         "chm_set_tuning": (i, [vp, i, vp]),
@@ -496,6 +498,13 @@ class Context:
         """(deflations, iteration graphs captured, graph launches) of this context's Davidson solves."""
         s = (C.c_int64 * 3)()
         self._check(self.lib.chm_davidson_stats(self.h, s), "chm_davidson_stats")
+        return tuple(s)
+
+    def split_stats(self):
+        """Centre sectors this context's Splits decomposed: (own kernels, rocSOLVER, own kernels
+        without convergence and then again rocSOLVER)."""
+        s = (C.c_int64 * 3)()
+        self._check(self.lib.chm_split_stats(self.h, s), "chm_split_stats")
         return tuple(s)
 
     def set_lower(self, veff):

@@ -2837,6 +2837,14 @@ int chm_davidson_stats(const chm_ctx* ctx, int64_t* out) {
   return CHM_OK;
 }
 
+int chm_split_stats(const chm_ctx* ctx, int64_t* out) {
+  if (!ctx || !out) return CHM_ERR_ARG;
+  out[0] = ctx->c.svd_own;
+  out[1] = ctx->c.svd_library;
+  out[2] = ctx->c.jacobi_retries;
+  return CHM_OK;
+}
+
 int chm_dmrg_nstates(const chm_ctx* ctx, int* n) {
   if (!ctx || !n) return CHM_ERR_ARG;
   *n = (int)ctx->c.lowers.size() + 1;

@@ -333,7 +333,9 @@ struct Ctx : HostState {
   int s_site = -1;
   void* rocblas = nullptr;  // rocblas_handle for the SVDs of Split
   static constexpr int SVD_STREAMS = 4;  // side streams of the large Split SVDs
-  int64_t jacobi_retries = 0;            // Jacobi sectors decomposed again by rocSOLVER (not converged)
+  // centre sectors decomposed by svd_batch, by rocSOLVER, and of the former again by rocSOLVER
+  // (not converged)
+  int64_t svd_own = 0, svd_library = 0, jacobi_retries = 0;
   int svd_max_sweeps = 0;                // CHM_SVD_MAX_SWEEPS: sweep limit of the Jacobi kernel (0: its own)
   // Split's matrices and workspaces, kept between calls (grown as needed)
   struct SplitWork {

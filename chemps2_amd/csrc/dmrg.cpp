@@ -334,6 +334,8 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     hip_check(hipStreamSynchronize(stream), "split SVD");
   };
   assemble_and_svd(std::vector<char>(cs.size(), 1));
+  for (const auto& c : cs)
+    if (c.cd > 0) (c.jac ? svd_own : svd_library)++;
   {
     // a Jacobi sector whose sweeps ended before every pair was orthogonal (the kernel's
     // info flag) is assembled again and decomposed by rocSOLVER's dgesvd, as the

@@ -117,6 +117,10 @@ int chm_s_set(chm_ctx* ctx, const double* x, int64_t n, int on_device);
  * site and site+1 with at most D states (change = 0 keeps the dimensions); needs the
  * FCI dimensions of chm_set_sectors_auto. The discarded weight goes to *disc_weight. */
 int chm_split(chm_ctx* ctx, int site, int D, int moving_right, int change, double* disc_weight);
+/* Centre sectors decomposed since the context was created: out[0] by the library's own
+ * kernels, out[1] by rocSOLVER, out[2] of those in out[0] that did not converge and were
+ * decomposed again by rocSOLVER. Measurement; no reference counterpart. */
+int chm_split_stats(const chm_ctx* ctx, int64_t* out);
 
 /* The whole DMRG on the device, mirroring CheMPS2::DMRG (DMRG.h:93-103): init =
  * SyBookkeeper(Prob, D) dimensions, a random left-normalised MPS from `seed`

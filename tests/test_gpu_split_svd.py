@@ -1,7 +1,8 @@
 """Split's decompositions at the sizes where its kernels change: panels of 16 columns, the
-one-workgroup Jacobi up to 64 columns, blocked rounds above it (block width 16, then
-narrower as the columns get longer), wide and tall sectors, rank deficiency, and the
-sectors longer than the in-house limit. One left and one right sector, so that all three
+Jacobi sweeps of one launch up to 32 columns and rounds of pairs of 16-column blocks above,
+wide and tall sectors, rank deficiency, and the sectors longer than the in-house limit. That
+the own kernels did it, and not the rocSOLVER call that repeats a sector without convergence,
+is read from the context's counters. One left and one right sector, so that all three
 centre sectors are a x b matrices of the test's choosing."""
 import numpy as np
 import pytest
@@ -67,5 +68,75 @@ def test_split_decompositions(a, b, rank):
         for q, two_sm in enumerate((0, 1, 0)):
             v = right[q * n * b:(q + 1) * n * b].reshape(b, n) / np.sqrt(two_sm + 1.0)
             assert np.abs(v.T @ v - np.eye(n)).max() <= tol
+    finally:
+        ctx.close()
+
+
+def boundaries(ctx, a, b):
+    """The three centre sectors of site 3 as a x b matrices."""
+    T, V = hubbard(8, U=3.0)
+    ctx.set_problem(8, 0, np.zeros(8, dtype=np.int32), 6, 0, 0, mx_table(T, V, 6))
+    ctx.set_sectors_auto(10 ** 6)
+    ctx.set_sectors(3, [(2, 0, 0, a)])
+    ctx.set_sectors(5, [(4, 0, 0, b)])
+    ctx.set_sectors(4, [(2, 0, 0, 1), (3, 1, 0, 1), (4, 0, 0, 1)])
+    for q in (3, 4):
+        ctx.mps_upload(q, np.ones(ctx.mps_layout_size(q)))
+    ctx.join(3)
+
+
+def graded(a, b, seed, rank=None):
+    """Centre matrices whose rows and columns fall over seven decades, and the object."""
+    rng = np.random.default_rng(seed)
+    parts = [rng.normal(size=(a, b)) * np.outer(10.0 ** (-3.5 * np.arange(a) / a), 10.0 ** (-3.5 * np.arange(b) / b))
+             for _ in range(3)]
+    if rank is not None:
+        r = max(1, int(rank * min(a, b)))
+        parts = [m[:, :r] @ rng.normal(size=(r, b)) for m in parts]
+    x = np.concatenate([parts[0].ravel("F"), parts[1].ravel("F"), np.zeros(a * b), parts[2].ravel("F")])
+    return parts, x / np.linalg.norm(x)
+
+
+def sides(ctx, a, b):
+    """(U, W = sigma V^T) of the three sectors after a Split to the right."""
+    n = min(a, b)
+    left, right = ctx.mps_download(3), ctx.mps_download(4)
+    return [(left[q * a * n:(q + 1) * a * n].reshape(n, a).T, right[q * n * b:(q + 1) * n * b].reshape(b, n).T)
+            for q in range(3)]
+
+
+@pytest.mark.parametrize("rank", [None, 0.4])
+@pytest.mark.parametrize("a,b", SIZES)
+def test_own_kernels_converge(a, b, rank):
+    print(f"case {a} x {b} rank {rank}", flush=True)
+    ctx = chemps2_amd.Context(0)
+    try:
+        boundaries(ctx, a, b)
+        ctx.s_set(graded(a, b, 1000 * a + b, rank)[1])
+        ctx.split(3, 10 ** 6, moving_right=True)
+        assert ctx.split_stats() == ((3, 0, 0) if max(a, b) <= 1024 else (0, 3, 0))
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("a,b", [(20, 30), (33, 40), (97, 130)])
+def test_sectors_without_convergence(monkeypatch, a, b):
+    # one sweep: up to 32 columns the kernel's own flag, above them the counters of the rounds
+    # say that the last sweep still rotated
+    print(f"case {a} x {b}, one sweep", flush=True)
+    monkeypatch.setenv("CHM_SVD_MAX_SWEEPS", "1")
+    ctx = chemps2_amd.Context(0)
+    try:
+        boundaries(ctx, a, b)
+        x = graded(a, b, a + b)[1]
+        ctx.s_set(x)
+        ctx.split(3, 10 ** 6, moving_right=True)
+        assert ctx.split_stats() == (3, 0, 3)
+        n = min(a, b)
+        tol = 10 * n * 2.0 ** -53
+        for u, _ in sides(ctx, a, b):
+            assert np.abs(u.T @ u - np.eye(n)).max() <= tol
+        ctx.join(3)
+        assert np.linalg.norm(ctx.s_get() - x) <= tol
     finally:
         ctx.close()
