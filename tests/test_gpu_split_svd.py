@@ -105,6 +105,40 @@ def sides(ctx, a, b):
             for q in range(3)]
 
 
+@pytest.mark.parametrize("scale", ["flat", "graded"])
+@pytest.mark.parametrize("a,b", [s for s in SIZES if max(s) <= 1024])
+def test_singular_vectors_orthonormal(a, b, scale):
+    # A column goes through n reflectors and some 10 n rotations, each of which rounds it by half
+    # a unit in the last place of its elements: a random walk of sqrt(11 n) such steps, of 0.5 x
+    # 2^-53 of its norm, twice in U^T U, for each of the n columns: 3.3 n 2^-53 in all where no
+    # rounding is systematic. The re-joined object, whose parts have their share of the norm:
+    # sqrt(11 n) of them.
+    print(f"case {a} x {b} {scale}", flush=True)
+    n = min(a, b)
+    parts, x = graded(a, b, 5 * a + b)
+    if scale == "flat":
+        rng = np.random.default_rng(5 * a + b)
+        x = np.concatenate([rng.normal(size=2 * a * b), np.zeros(a * b), rng.normal(size=a * b)])
+        x /= np.linalg.norm(x)
+    ctx = chemps2_amd.Context(0)
+    try:
+        boundaries(ctx, a, b)
+        ctx.s_set(x)
+        ctx.split(3, 10 ** 6, moving_right=True)
+        us = [u for u, _ in sides(ctx, a, b)]
+        ctx.join(3)
+        error = np.linalg.norm(ctx.s_get() - x)
+        ctx.s_set(x)
+        ctx.split(3, 10 ** 6, moving_right=False)
+        vs = [w.T / np.sqrt(q % 2 + 1.0) for q, (_, w) in enumerate(sides(ctx, a, b))]
+        loss = max(np.linalg.norm(m.T @ m - np.eye(n)) for m in us + vs) * 2.0 ** 53
+        print(f"  {loss / n:.2f} n, {error * 2.0 ** 53 / np.sqrt(n):.2f} sqrt(n) units", flush=True)
+        assert loss <= 6 * max(n, 2)
+        assert error * 2.0 ** 53 <= 2 * np.sqrt(11 * max(n, 2))
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("rank", [None, 0.4])
 @pytest.mark.parametrize("a,b", SIZES)
 def test_own_kernels_converge(a, b, rank):
