@@ -405,7 +405,8 @@ struct DevSvd {
   double* U;
   double* VT;
   double* S;
-  double* floor2;  // norm^2 at or below which a column is numerically zero
+  double* floor2;  // norm^2 at or below which a column is numerically zero; the power of two that
+                   // brings the sector to order one
   int* perm;       // n
   int* src;        // n
   int* rot;        // SVD_SWEEPS: workgroups that rotated, by sweep (more than 32 columns)
@@ -413,6 +414,7 @@ struct DevSvd {
   int m, n;
   int wide;
   int max_sweeps;  // at most SVD_SWEEPS
+  int sector;      // the caller's number of it
 };
 constexpr int SVD_SWEEPS = 40;      // sweep limit
 constexpr int SVD_ALONE = 32;       // sectors up to this width run all sweeps in one launch

@@ -216,7 +216,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   Xw.alloc(std::max<int64_t>(qsz, 1));
   Jw.alloc(std::max<int64_t>(qsz, 1));
   Tw.alloc(std::max<int64_t>(tsz, 1));
-  Fw.alloc(std::max<int64_t>(nsec, 1));
+  Fw.alloc(std::max<int64_t>(2 * nsec, 1));
   Iw.alloc(std::max<int64_t>(2 * ssz, 1));
   Rw.alloc(std::max<int64_t>(nsec * SVD_SWEEPS, 1));
   std::vector<int> h_rot(std::max<int64_t>(nsec * SVD_SWEEPS, 1), 0);
@@ -282,7 +282,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
         DevSvd j{};
         j.A = M.p + c.moff; j.W = Ww.p + c.moff; j.X = Xw.p + c.qoff; j.J = Jw.p + c.qoff; j.T = Tw.p + c.toff;
         j.U = U.p + c.uoff; j.VT = VT.p + c.voff; j.S = Sg.p + c.soff;
-        j.floor2 = Fw.p + q; j.perm = Iw.p + 2 * c.soff; j.src = Iw.p + 2 * c.soff + c.cd;
+        j.floor2 = Fw.p + 2 * q; j.sector = (int)q; j.perm = Iw.p + 2 * c.soff; j.src = Iw.p + 2 * c.soff + c.cd;
         j.info = info.p + q;
         j.m = std::max(c.dLt, c.dRt); j.n = c.cd; j.wide = c.dLt < c.dRt;
         j.rot = Rw.p + (int64_t)SVD_SWEEPS * js.size();
@@ -346,7 +346,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     std::vector<char> redo(cs.size(), 0);
     bool any = false;
     for (const DevSvd& j : jobs)  // wider sectors: the last sweep allowed still rotated
-      if (j.n > SVD_ALONE && h_rot[(j.rot - Rw.p) + j.max_sweeps - 1] != 0) inf[j.floor2 - Fw.p] = 1;
+      if (j.n > SVD_ALONE && h_rot[(j.rot - Rw.p) + j.max_sweeps - 1] != 0) inf[j.sector] = 1;
     for (size_t q = 0; q < cs.size(); q++) {
       if (inf[q] == 0) continue;
       if (!cs[q].jac) throw Error{ERR_NUMERIC, "SVD did not converge"};
@@ -410,7 +410,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     // vectors of zero singular values that are kept: completed to orthonormal sets
     std::vector<DevSvd> zero;
     for (const DevSvd& j : jobs) {
-      const Center& c = cs[j.floor2 - Fw.p];
+      const Center& c = cs[j.sector];
       const int lim = std::min(sec.dim(st + 1, c.nm, c.sm, c.im), c.cd);
       if (c.jac && lim > 0 && sv[c.soff + lim - 1] == 0.0) zero.push_back(j);
     }

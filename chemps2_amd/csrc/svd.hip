@@ -74,42 +74,89 @@ __device__ __forceinline__ void pair_of(int n2, int r, int k, int& p, int& q) {
   if (p > q) { const int t = p; p = q; q = t; }
 }
 
-// Column norms of A, their order (perm: sorted position -> column), the floor, counters
-// cleared. One workgroup per sector.
+// The largest element's magnitude for the whole workgroup (SVD_INF when one is not finite).
+constexpr double SVD_INF = __builtin_huge_val();
+__device__ double max_abs(const double* __restrict__ a, int n, int tid, double* red) {
+  double mx = 0.0;
+  for (int e = tid; e < n; e += JT) {
+    const double v = fabs(a[e]);
+    mx = v <= 1.7976931348623157e308 ? fmax(mx, v) : SVD_INF;
+    if (mx == SVD_INF) break;
+  }
+  red[tid] = mx;
+  __syncthreads();
+  for (int h = JT / 2; h > 0; h >>= 1) {
+    if (tid < h) red[tid] = fmax(red[tid], red[tid + h]);
+    __syncthreads();
+  }
+  mx = red[0];
+  __syncthreads();
+  return mx;
+}
+
+// The power of two that brings the sector to order one, column norms of A so scaled, their order
+// (perm: sorted position -> column), the floor, counters cleared. One workgroup per sector. The
+// rotations multiply squared norms, which takes them out of the range of doubles for columns
+// below 1e-80 or above 1e77; the scale comes from the sum of the squares, or from the largest
+// element where the squares themselves leave that range. A sector with an element that is
+// not finite counts as zero (scale 0).
 __global__ __launch_bounds__(JT) void k_svd_sort(const DevSvd* __restrict__ jobs) {
-  __shared__ double nrm[SVD_MAXM];
+  __shared__ double nrm[SVD_MAXM], red[JT];
   const DevSvd it = jobs[blockIdx.x];
   const int m = it.m, n = it.n, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int j = wv; j < n; j += JW) {
+  auto norms = [&](double scale) {  // and the sum of their squares
+    for (int j = wv; j < n; j += JW) {
+      double s = 0.0;
+      for (int i = lane; i < m; i += 64) {
+        const double v = it.A[i + (size_t)m * j] * scale;
+        s = fma(v, v, s);
+      }
+      s = wave_sum(s);
+      if (lane == 0) nrm[j] = s;
+    }
+    __syncthreads();
     double s = 0.0;
-    for (int i = lane; i < m; i += 64) s = fma(it.A[i + (size_t)m * j], it.A[i + (size_t)m * j], s);
-    s = wave_sum(s);
-    if (lane == 0) nrm[j] = s == s ? s : 0.0;
+    for (int j = lane; j < n; j += 64) s += nrm[j];
+    return wave_sum(s);
+  };
+  double sum = norms(1.0), scale, unit = 1.0;  // unit: the scale of nrm and sum
+  if (sum > 1e-200 && sum < 1e200) {
+    scale = ldexp(1.0, -ilogb(sum) / 2);
+  } else {
+    const double mx = max_abs(it.A, m * n, tid, red);
+    if (mx > 0.0 && mx < SVD_INF) {
+      scale = unit = ldexp(1.0, max(-1000, min(1000, -ilogb(mx))));
+      sum = norms(unit);
+    } else {
+      scale = mx > 0.0 ? 0.0 : 1.0;
+      sum = 0.0;
+      for (int j = tid; j < n; j += JT) nrm[j] = 0.0;
+      __syncthreads();
+    }
   }
-  __syncthreads();
   for (int j = tid; j < n; j += JT) {
     int r = 0;
     for (int k = 0; k < n; k++) r += (nrm[k] > nrm[j] || (nrm[k] == nrm[j] && k < j)) ? 1 : 0;
     it.perm[r] = j;
   }
-  if (wv == JW - 1) {
-    double s = 0.0;
-    for (int j = lane; j < n; j += 64) s += nrm[j];
-    s = wave_sum(s);
-    if (lane == 0) *it.floor2 = SVD_EPS * SVD_EPS * s;
+  if (tid == JT - 1) {
+    const double f = unit == scale ? 1.0 : scale;
+    it.floor2[0] = SVD_EPS * SVD_EPS * (sum * f * f);
+    it.floor2[1] = scale;
   }
   for (int q = tid; q < SVD_SWEEPS; q += JT) it.rot[q] = 0;
   if (tid == 0) *it.info = 0;
 }
 
-// W = A in sorted order, X cleared, J the identity; SVD_CHUNKS workgroups per sector.
+// W = A in sorted order and scaled, X cleared, J the identity; SVD_CHUNKS workgroups per sector.
 constexpr int SVD_CHUNKS = 16;
 __global__ __launch_bounds__(QT) void k_svd_copy(const DevSvd* __restrict__ jobs) {
   const DevSvd it = jobs[blockIdx.y];
   const int m = it.m, n = it.n, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const double scale = it.floor2[1];
   for (int t = blockIdx.x * QW + wv; t < n; t += SVD_CHUNKS * QW) {
     const double* a = it.A + (size_t)m * it.perm[t];
-    for (int i = lane; i < m; i += 64) it.W[i + (size_t)m * t] = a[i];
+    for (int i = lane; i < m; i += 64) it.W[i + (size_t)m * t] = scale == 0.0 ? 0.0 : a[i] * scale;
     for (int i = lane; i < n; i += 64) {
       it.X[i + (size_t)n * t] = 0.0;
       it.J[i + (size_t)n * t] = i == t ? 1.0 : 0.0;
@@ -295,20 +342,21 @@ __device__ __forceinline__ void times_rotations(double* X, double* J, int n, con
 // The rotation that makes columns of norms^2 al, be and dot product ga orthogonal, as s = sin
 // and h = tan of its half angle, or (0, 0) when |ga| <= tol sqrt(al be) (the rounding floor of
 // the dot product, the stopping rule of LAPACK's dgesvj) or a norm is at most the floor fl
-// (numerically zero). The angle and the test come from the hardware's approximate reciprocal and
-// roots (2^29 units in the last place: what is left of ga is that much smaller, which costs no
-// sweep); s is refined to full precision for the h that came out, so the rotation is
-// orthogonal whatever the angle.
+// (numerically zero); tol2 is tol^2. The angle comes from the hardware's approximate reciprocal
+// and roots (2^29 units in the last place: what is left of ga is that much smaller, which costs
+// no sweep); s is refined to full precision for the h that came out, so the rotation is
+// orthogonal whatever the angle. The sector is of order one and columns below its floor stay as they
+// are, so al and be lie between 1e-33 and 1e7 and no product comes near the limits of doubles.
 struct Rot {
   double s, h;
 };
-__device__ __forceinline__ Rot rotation(double al, double be, double ga, double tol, double fl) {
+__device__ __forceinline__ Rot rotation(double al, double be, double ga, double tol2, double fl) {
   const double d = be - al, r = __builtin_amdgcn_sqrt(fma(d, d, 4.0 * ga * ga));
   const double t = (d >= 0.0 ? 2.0 : -2.0) * ga * __builtin_amdgcn_rcp(fabs(d) + r);
   const double c = __builtin_amdgcn_rsq(fma(t, t, 1.0)), h = t * c * __builtin_amdgcn_rcp(1.0 + c);
   // 1 / (1 + h^2) = (1 + cos) / 2
   const double q = fma(0.5, c, 0.5), e = fma(-fma(h, h, 1.0), q, 1.0);
-  const bool on = al > fl && be > fl && fabs(ga) * __builtin_amdgcn_rsq(al) * __builtin_amdgcn_rsq(be) > tol;
+  const bool on = al > fl && be > fl && ga * ga > tol2 * (al * be);
   return on ? Rot{2.0 * h * fma(q, fma(e, e, e), q), h} : Rot{0.0, 0.0};
 }
 // (u, v) <- (c u - s v, s u + c v), with c = 1 - s h: what rounding and an s that is not quite
@@ -341,7 +389,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   if (wq == 0 && r > 0) return;
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const double fl = *it.floor2, tol = sqrt((double)n + 30.0) * SVD_EPS;
+  const double fl = it.floor2[0], tol2 = ((double)n + 30.0) * (SVD_EPS * SVD_EPS);
   for (;;) {
     {  // Gram matrix: [p p], [p q], [q q] blocks, rows dealt out to the wavefronts
       svd_t4 a0 = {0.0, 0.0, 0.0, 0.0}, a1 = a0, a2 = a0;
@@ -387,7 +435,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     for (int e = tid; e < 1024; e += RT) {
       const int i = e >> 5, j = e & 31;
       if (i >= j || (r > 0 && (i >= 16 || j < 16))) continue;
-      if (rotation(g[0][i * 34], g[0][j * 34], g[0][i * 33 + j], tol, fl).s != 0.0) rotated = 1;
+      if (rotation(g[0][i * 34], g[0][j * 34], g[0][i * 33 + j], tol2, fl).s != 0.0) rotated = 1;
     }
     __syncthreads();
     if (!rotated) break;
@@ -405,11 +453,11 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
       };
       int u, v;
       slots(pb, u, v);
-      const Rot rb = rotation(gi[u * 34], gi[v * 34], gi[u * 33 + v], tol, fl);
+      const Rot rb = rotation(gi[u * 34], gi[v * 34], gi[u * 33 + v], tol2, fl);
       if (tid < 256) {  // G <- R^T G R, a 2 x 2 block per thread
         int x, y;
         slots(pa, x, y);
-        const Rot ra = rotation(gi[x * 34], gi[y * 34], gi[x * 33 + y], tol, fl);
+        const Rot ra = rotation(gi[x * 34], gi[y * 34], gi[x * 33 + y], tol2, fl);
         double x1, x2, y1, y2;
         rotate(rb, gi[x * 33 + u], gi[x * 33 + v], x1, x2);
         rotate(rb, gi[y * 33 + u], gi[y * 33 + v], y1, y2);
@@ -434,13 +482,13 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   }
 }
 
-// Singular values (the norms of X's columns, zero below the floor) in falling order and
-// their columns (src).
+// Singular values of the scaled sector (the norms of X's columns, zero below the floor) in
+// falling order and their columns (src).
 __global__ __launch_bounds__(JT) void k_svd_sigma(const DevSvd* __restrict__ jobs) {
   __shared__ double sig[SVD_MAXM];
   const DevSvd it = jobs[blockIdx.x];
   const int n = it.n, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const double fl = *it.floor2;
+  const double fl = it.floor2[0];
   for (int j = wv; j < n; j += JW) {
     double s = 0.0;
     for (int i = lane; i < n; i += 64) s = fma(it.X[i + (size_t)n * j], it.X[i + (size_t)n * j], s);
@@ -457,7 +505,7 @@ __global__ __launch_bounds__(JT) void k_svd_sigma(const DevSvd* __restrict__ job
 }
 
 // The n-long singular vectors, 16 per workgroup: row perm[i] of vector t is X[i, src[t]] /
-// sigma_t (zero for sigma_t = 0). VT is written 16 neighbouring t at a time.
+// sigma_t (zero for sigma_t = 0), sigma still scaled. VT is written 16 neighbouring t at a time.
 __global__ __launch_bounds__(QT) void k_svd_short(const DevSvd* __restrict__ jobs) {
   const DevSvd it = jobs[blockIdx.y];
   const int n = it.n, t0 = PB * blockIdx.x;
@@ -480,7 +528,8 @@ __global__ __launch_bounds__(QT) void k_svd_short(const DevSvd* __restrict__ job
 
 // The m-long singular vectors Q J, 16 of them per workgroup: the columns src[t] of J padded
 // to m rows (or, to complete a basis, the unit vectors e_t), in LDS, through the panels'
-// reflectors in falling order (I - V T V^T). complete: only the vectors with sigma_t = 0.
+// reflectors in falling order (I - V T V^T). complete: only the vectors with sigma_t = 0; else the
+// singular values also lose their scale.
 __global__ __launch_bounds__(QT) void k_svd_long(const DevSvd* __restrict__ jobs, int complete) {
   extern __shared__ double P[];  // 16 columns of m
   __shared__ double part[QW][256];
@@ -489,6 +538,7 @@ __global__ __launch_bounds__(QT) void k_svd_long(const DevSvd* __restrict__ jobs
   const int m = it.m, n = it.n, nb = (n + PB - 1) / PB, t0 = PB * blockIdx.x;
   if (t0 >= n) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lg = lane >> 4;
+  if (!complete && tid < PB && t0 + tid < n && it.floor2[1] > 0.0) it.S[t0 + tid] *= 1.0 / it.floor2[1];
   for (int c = wv; c < PB; c += QW) {
     const int t = t0 + c;
     const double* x = it.J + (t < n && !complete ? (size_t)n * it.src[t] : 0);

@@ -139,6 +139,57 @@ def test_singular_vectors_orthonormal(a, b, scale):
         ctx.close()
 
 
+@pytest.mark.parametrize("scale", [1e-90, 1e-159, 1e-290, 1e90, 1e160])
+@pytest.mark.parametrize("a,b", [(6, 6), (24, 40), (70, 50)])
+def test_sectors_of_any_magnitude(a, b, scale):
+    # a sector far from order one, whose norms to the second or fourth power leave the range of
+    # doubles, beside two of order one
+    print(f"case {a} x {b} scale {scale}", flush=True)
+    n = min(a, b)
+    _, x = graded(a, b, a + b)
+    x[:a * b] *= scale
+    ctx = chemps2_amd.Context(0)
+    try:
+        boundaries(ctx, a, b)
+        ctx.s_set(x)
+        ctx.split(3, 10 ** 6, moving_right=True)
+        assert ctx.split_stats() == (3, 0, 0)
+        tol = 10 * n * 2.0 ** -53
+        for u, _ in sides(ctx, a, b):
+            assert np.abs(u.T @ u - np.eye(n)).max() <= tol
+        ctx.join(3)
+        for got, ref in zip(ctx.s_get().reshape(4, -1), x.reshape(4, -1)):
+            big = np.abs(ref).max() or 1.0
+            assert np.linalg.norm(got / big - ref / big) <= tol * np.linalg.norm(ref / big)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("a,b", [(6, 6), (24, 40), (70, 50)])
+def test_sector_without_finite_values(a, b, bad):
+    # such a sector counts as zero: sigma = 0 and orthonormal vectors; the others are untouched
+    print(f"case {a} x {b} {bad}", flush=True)
+    n = min(a, b)
+    _, x = graded(a, b, a + b)
+    y = x.copy()
+    y[a * b // 2] = bad
+    ctx = chemps2_amd.Context(0)
+    try:
+        boundaries(ctx, a, b)
+        ctx.s_set(y)
+        ctx.split(3, 10 ** 6, moving_right=True)
+        assert ctx.split_stats() == (3, 0, 0)
+        tol = 10 * n * 2.0 ** -53
+        for u, _ in sides(ctx, a, b):
+            assert np.abs(u.T @ u - np.eye(n)).max() <= tol
+        assert not sides(ctx, a, b)[0][1].any()
+        ctx.join(3)
+        assert np.linalg.norm(ctx.s_get()[a * b:] - x[a * b:]) <= tol
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("rank", [None, 0.4])
 @pytest.mark.parametrize("a,b", SIZES)
 def test_own_kernels_converge(a, b, rank):
