@@ -340,13 +340,14 @@ __device__ __forceinline__ void times_rotations(double* X, double* J, int n, con
 }
 
 // The rotation that makes columns of norms^2 al, be and dot product ga orthogonal, as s = sin
-// and h = tan of its half angle, or (0, 0) when |ga| <= tol sqrt(al be) (the rounding floor of
-// the dot product, the stopping rule of LAPACK's dgesvj) or a norm is at most the floor fl
-// (numerically zero); tol2 is tol^2. The angle comes from the hardware's approximate reciprocal
-// and roots (2^29 units in the last place: what is left of ga is that much smaller, which costs
-// no sweep); s is refined to full precision for the h that came out, so the rotation is
-// orthogonal whatever the angle. The sector is of order one and columns below its floor stay as they
-// are, so al and be lie between 1e-33 and 1e7 and no product comes near the limits of doubles.
+// and h = tan of its half angle, or (0, 0) when |ga| <= tol sqrt(al be), tol = sqrt(n) 2^-53
+// (the rounding floor of the dot product, the stopping rule of LAPACK's dgesvj), or a norm is
+// at most the floor fl (numerically zero); tol2 is tol^2. The angle comes from the hardware's
+// approximate reciprocal and roots (2^29 units in the last place: what is left of ga is that much
+// smaller, which costs no sweep); s is refined to full precision for the h that came out, so the
+// rotation is orthogonal whatever the angle. The sector is of order one and columns below its
+// floor stay as they are, so al and be lie between 1e-33 and 1e7 and no product comes near the
+// limits of doubles.
 struct Rot {
   double s, h;
 };
@@ -389,7 +390,7 @@ __global__ __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   if (wq == 0 && r > 0) return;
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const double fl = it.floor2[0], tol2 = ((double)n + 30.0) * (SVD_EPS * SVD_EPS);
+  const double fl = it.floor2[0], tol2 = (double)n * (SVD_EPS * SVD_EPS);
   for (;;) {
     {  // Gram matrix: [p p], [p q], [q q] blocks, rows dealt out to the wavefronts
       svd_t4 a0 = {0.0, 0.0, 0.0, 0.0}, a1 = a0, a2 = a0;

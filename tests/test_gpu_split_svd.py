@@ -139,6 +139,31 @@ def test_singular_vectors_orthonormal(a, b, scale):
         ctx.close()
 
 
+@pytest.mark.parametrize("n", [2, 3, 5, 8])
+def test_small_sectors_stop_at_the_rounding_floor(n):
+    # the sweeps end with no pair of columns above sqrt(n) 2^-53; normalising them adds a rounding
+    # of half a unit to each element
+    print(f"case {n} x {n}", flush=True)
+    worst = 0.0
+    ctx = chemps2_amd.Context(0)
+    try:
+        boundaries(ctx, n, n)
+        for seed in range(60):
+            if seed > 0:
+                ctx.join(3)
+            x = np.random.default_rng(seed).normal(size=4 * n * n)
+            x[2 * n * n:3 * n * n] = 0.0
+            ctx.s_set(x)
+            ctx.split(3, 10 ** 6, moving_right=False)
+            for q, (_, w) in enumerate(sides(ctx, n, n)):
+                v = (w / np.sqrt(q % 2 + 1.0)).astype(np.longdouble)
+                worst = max(worst, float(np.abs(np.triu(v @ v.T, 1)).max()) * 2.0 ** 53)
+        print(f"  {worst:.2f} units", flush=True)
+        assert worst <= np.sqrt(n) + 1.5
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("scale", [1e-90, 1e-159, 1e-290, 1e90, 1e160])
 @pytest.mark.parametrize("a,b", [(6, 6), (24, 40), (70, 50)])
 def test_sectors_of_any_magnitude(a, b, scale):
