@@ -418,7 +418,8 @@ struct DevSvd {
 };
 constexpr int SVD_SWEEPS = 40;      // sweep limit
 constexpr int SVD_ALONE = 32;       // sectors up to this width run all sweeps in one launch
-constexpr int SVD_MAXM = 1024;      // longest sector: a QR panel of 16 columns in LDS
+constexpr int SVD_MAXM = 1024;      // longest sector with a QR panel of 16 columns in LDS; widest
+constexpr int SVD_TALLM = 4096, SVD_TALLN = 256;  // longest and widest with the panels in memory
 template <class T>
 struct DBuf;
 // Decomposes all jobs (sorted by falling n); buf holds their device copy. d_rot: the jobs'

@@ -165,7 +165,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   struct Mult { int n, s, i, d; };
   struct Center {
     int nm, sm, im, dLt = 0, dRt = 0, cd = 0;
-    bool jac = false;  // svd_batch or rocSOLVER (sectors longer than SVD_MAXM)
+    bool jac = false;  // svd_batch or rocSOLVER
     int64_t moff = 0, uoff = 0, voff = 0, soff = 0, qoff = 0, toff = 0;
     std::vector<Mult> lf, rt;
   };
@@ -197,7 +197,11 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   int64_t msz = 0, usz = 0, vsz = 0, ssz = 0, qsz = 0, tsz = 0;
   for (auto& c : cs) {
     if (c.cd <= 0) continue;
-    c.jac = c.cd <= svd_jacobi_maxn && std::max(c.dLt, c.dRt) <= SVD_MAXM;
+    // Longer sectors, those of steps near the chain's ends, have their QR panels in memory instead
+    // of LDS, up to 4096 x 256 (three of 2000 x 250: 10.4 ms, 62 ms by rocSOLVER's gesvdj; of
+    // 1100 x 200: 5.8 and 56 ms; the error of the re-joined object 3e-15 to 4e-15 and 6e-14 to 7e-14)
+    const int m = std::max(c.dLt, c.dRt);
+    c.jac = c.cd <= svd_jacobi_maxn && (m <= SVD_MAXM || (m <= SVD_TALLM && c.cd <= SVD_TALLN));
     c.moff = msz; msz += (int64_t)c.dLt * c.dRt;
     c.uoff = usz; usz += (int64_t)c.dLt * c.cd;
     c.voff = vsz; vsz += (int64_t)c.cd * c.dRt;
@@ -229,8 +233,8 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   info.alloc(std::max<size_t>(cs.size(), 1));
   hip_check(hipMemsetAsync(info.p, 0, std::max<size_t>(cs.size(), 1) * sizeof(rocblas_int), stream), "clear info");
   // Assembly and SVD of the selected sectors (sel[q]): the centre matrices from the S
-  // blocks with their recoupling factors, then svd_batch for the sectors of at most
-  // SVD_MAXM rows and columns and rocSOLVER for the others.
+  // blocks with their recoupling factors, then svd_batch for the sectors within its limits
+  // and rocSOLVER for the others.
   auto assemble_and_svd = [&](const std::vector<char>& sel) {
     std::vector<DevCopy> items;
     for (size_t q = 0; q < cs.size(); q++) {

@@ -178,15 +178,17 @@ __device__ __forceinline__ void sum_parts(const double (*part)[256], double* out
 // k - 1 (I - V T^T V^T), whose rows of R then go to X = R^T; the workgroup of block k also
 // factors it as the next panel: V (unit lower trapezoidal, zeros above) to A, T to T, its R
 // to X. The products are 16 x 16 results on the matrix cores, rows dealt out to the
-// wavefronts; the panel is in LDS.
+// wavefronts; the panel is in LDS, or (TALL: sectors of more than SVD_MAXM rows, the others in
+// the launch without TALL) factored where it lies, in W.
+template <bool TALL>
 __global__ __launch_bounds__(QT) void k_qr_step(const DevSvd* __restrict__ jobs, int k) {
-  extern __shared__ double P[];  // panel: column c at P + c mk
+  extern __shared__ double panel[];
   __shared__ double part[QW][256];
   __shared__ double w1[256], w2[256];
   __shared__ double tau[PB], scl[PB], bet[PB];
   const DevSvd it = jobs[blockIdx.y];
   const int m = it.m, n = it.n, nb = (n + PB - 1) / PB, j = k + (int)blockIdx.x;
-  if (j >= nb) return;
+  if (j >= nb || (m > SVD_MAXM) != TALL) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lg = lane >> 4;
   const int c0 = PB * j, cw = min(PB, n - c0);
   double* C = it.W + (size_t)m * c0;
@@ -239,15 +241,22 @@ __global__ __launch_bounds__(QT) void k_qr_step(const DevSvd* __restrict__ jobs,
   }
   if (j != k) return;
   const int q0 = PB * k, mk = m - q0;
+  double* P;         // panel: column c at P + c ps
+  const int ps = TALL ? m : mk;
   __syncthreads();
-  for (int c = wv; c < PB; c += QW)
-    for (int i = lane; i < mk; i += 64) P[c * mk + i] = c < cw ? C[q0 + i + (size_t)m * c] : 0.0;
-  __syncthreads();
+  if constexpr (TALL) {
+    P = C + q0;
+  } else {
+    P = panel;
+    for (int c = wv; c < PB; c += QW)
+      for (int i = lane; i < mk; i += 64) P[c * ps + i] = c < cw ? C[q0 + i + (size_t)m * c] : 0.0;
+    __syncthreads();
+  }
   for (int c = 0; c < cw; c++) {
     double s = 0.0;
-    for (int i = c + 1 + lane; i < mk; i += 64) s = fma(P[c * mk + i], P[c * mk + i], s);
+    for (int i = c + 1 + lane; i < mk; i += 64) s = fma(P[c * ps + i], P[c * ps + i], s);
     s = wave_sum(s);
-    const double a = P[c * mk + c];
+    const double a = P[c * ps + c];
     double tc = 0.0, sc = 0.0, bc = a;
     if (s > 0.0) {
       bc = a >= 0.0 ? -sqrt(fma(a, a, s)) : sqrt(fma(a, a, s));
@@ -257,25 +266,25 @@ __global__ __launch_bounds__(QT) void k_qr_step(const DevSvd* __restrict__ jobs,
     if (tid == 0) { tau[c] = tc; scl[c] = sc; bet[c] = bc; }
     for (int q = c + 1 + wv; q < cw; q += QW) {
       double d = 0.0;
-      for (int i = c + 1 + lane; i < mk; i += 64) d = fma(P[c * mk + i], P[q * mk + i], d);
-      d = tc * fma(sc, wave_sum(d), P[q * mk + c]);
+      for (int i = c + 1 + lane; i < mk; i += 64) d = fma(P[c * ps + i], P[q * ps + i], d);
+      d = tc * fma(sc, wave_sum(d), P[q * ps + c]);
       const double ds = d * sc;
-      for (int i = c + 1 + lane; i < mk; i += 64) P[q * mk + i] = fma(-ds, P[c * mk + i], P[q * mk + i]);
-      if (lane == 0) P[q * mk + c] -= d;
+      for (int i = c + 1 + lane; i < mk; i += 64) P[q * ps + i] = fma(-ds, P[c * ps + i], P[q * ps + i]);
+      if (lane == 0) P[q * ps + c] -= d;
     }
     __syncthreads();
   }
   for (int e = tid; e < 256; e += QT) {
     const int i = e & 15, c = e >> 4;
-    if (c < cw && i <= c) it.X[c0 + c + (size_t)n * (c0 + i)] = i < c ? P[c * mk + i] : bet[c];
+    if (c < cw && i <= c) it.X[c0 + c + (size_t)n * (c0 + i)] = i < c ? P[c * ps + i] : bet[c];
   }
   __syncthreads();
   for (int c = wv; c < cw; c += QW) {
     double* V = it.A + (size_t)m * (c0 + c);
     for (int i = lane; i < q0; i += 64) V[i] = 0.0;
     for (int i = lane; i < mk; i += 64) {
-      const double v = i < c ? 0.0 : (i == c ? 1.0 : scl[c] * P[c * mk + i]);
-      P[c * mk + i] = v;
+      const double v = i < c ? 0.0 : (i == c ? 1.0 : scl[c] * P[c * ps + i]);
+      P[c * ps + i] = v;
       V[q0 + i] = v;
     }
   }
@@ -283,7 +292,7 @@ __global__ __launch_bounds__(QT) void k_qr_step(const DevSvd* __restrict__ jobs,
   {  // V^T V, then T by columns: T(0:c, c) = -tau_c T(0:c, 0:c) V^T v_c
     svd_t4 acc = {0.0, 0.0, 0.0, 0.0};
     for (int base = 4 * wv; base < mk; base += 4 * QW) {
-      const double v = base + lg < mk ? P[lr * mk + base + lg] : 0.0;
+      const double v = base + lg < mk && (!TALL || lr < cw) ? P[lr * ps + base + lg] : 0.0;
       acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, acc, 0, 0, 0);
     }
 #pragma unroll
@@ -530,17 +539,23 @@ __global__ __launch_bounds__(QT) void k_svd_short(const DevSvd* __restrict__ job
 // The m-long singular vectors Q J, 16 of them per workgroup: the columns src[t] of J padded
 // to m rows (or, to complete a basis, the unit vectors e_t), in LDS, through the panels'
 // reflectors in falling order (I - V T V^T). complete: only the vectors with sigma_t = 0; else the
-// singular values also lose their scale.
+// singular values also lose their scale. TALL (as in k_qr_step): the vectors in their columns
+// of W, which the factorisation left free, instead of LDS.
+template <bool TALL>
 __global__ __launch_bounds__(QT) void k_svd_long(const DevSvd* __restrict__ jobs, int complete) {
-  extern __shared__ double P[];  // 16 columns of m
+  extern __shared__ double panel[];
   __shared__ double part[QW][256];
   __shared__ double w1[256], w2[256];
   const DevSvd it = jobs[blockIdx.y];
   const int m = it.m, n = it.n, nb = (n + PB - 1) / PB, t0 = PB * blockIdx.x;
-  if (t0 >= n) return;
+  if (t0 >= n || (m > SVD_MAXM) != TALL) return;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lr = lane & 15, lg = lane >> 4;
+  const int tw = TALL ? min(PB, n - t0) : PB;  // columns of P
+  double* P;                                   // 16 columns of m
+  if constexpr (TALL) P = it.W + (size_t)m * t0;
+  else P = panel;
   if (!complete && tid < PB && t0 + tid < n && it.floor2[1] > 0.0) it.S[t0 + tid] *= 1.0 / it.floor2[1];
-  for (int c = wv; c < PB; c += QW) {
+  for (int c = wv; c < tw; c += QW) {
     const int t = t0 + c;
     const double* x = it.J + (t < n && !complete ? (size_t)n * it.src[t] : 0);
     for (int i = lane; i < m; i += 64)
@@ -558,7 +573,7 @@ __global__ __launch_bounds__(QT) void k_svd_long(const DevSvd* __restrict__ jobs
       for (int s = 0; s < 4; s++) {
         const int row = base + 4 * lg + s;
         v[s] = (row < m && lr < cw) ? V[row + (size_t)m * lr] : 0.0;
-        c[s] = row < m ? P[lr * m + row] : 0.0;
+        c[s] = (row < m && lr < tw) ? P[lr * m + row] : 0.0;
       }
 #pragma unroll
       for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v[s], c[s], acc, 0, 0, 0);
@@ -585,7 +600,7 @@ __global__ __launch_bounds__(QT) void k_svd_long(const DevSvd* __restrict__ jobs
       }
 #pragma unroll
       for (int r = 0; r < 4; r++)
-        if (row < m) P[(4 * r + lg) * m + row] -= d[r];
+        if (row < m && 4 * r + lg < tw) P[(4 * r + lg) * m + row] -= d[r];
     }
     __syncthreads();
   }
@@ -617,21 +632,37 @@ size_t qr_lds(int m) { return (size_t)PB * m * sizeof(double); }
 
 // the LDS of the QR kernels
 void svd_setup() {
-  hip_check(hipFuncSetAttribute((const void*)k_qr_step, hipFuncAttributeMaxDynamicSharedMemorySize, (int)qr_lds(SVD_MAXM)), "SVD kernel LDS");
-  hip_check(hipFuncSetAttribute((const void*)k_svd_long, hipFuncAttributeMaxDynamicSharedMemorySize, (int)qr_lds(SVD_MAXM)), "SVD kernel LDS");
+  hip_check(hipFuncSetAttribute((const void*)k_qr_step<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)qr_lds(SVD_MAXM)), "SVD kernel LDS");
+  hip_check(hipFuncSetAttribute((const void*)k_svd_long<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)qr_lds(SVD_MAXM)), "SVD kernel LDS");
 }
 
-void launch_qr(const DevSvd* d, const std::vector<DevSvd>& jobs, hipStream_t s) {
+// panels of the widest sector, rows of the longest with its panel in LDS (0: none), any longer
+struct Extent {
   int nb = 0, m = 0;
-  for (const DevSvd& j : jobs) { nb = std::max(nb, (j.n + PB - 1) / PB); m = std::max(m, j.m); }
-  for (int k = 0; k < nb; k++)
-    hipLaunchKernelGGL(k_qr_step, dim3(nb - k, (int)jobs.size()), dim3(QT), qr_lds(m), s, d, k);
+  bool tall = false;
+  explicit Extent(const std::vector<DevSvd>& jobs) {
+    for (const DevSvd& j : jobs) {
+      nb = std::max(nb, (j.n + PB - 1) / PB);
+      if (j.m > SVD_MAXM) tall = true;
+      else m = std::max(m, j.m);
+    }
+  }
+};
+
+void launch_qr(const DevSvd* d, const std::vector<DevSvd>& jobs, hipStream_t s) {
+  const Extent x(jobs);
+  for (int k = 0; k < x.nb; k++) {
+    const dim3 grid(x.nb - k, (int)jobs.size());
+    if (x.m > 0) hipLaunchKernelGGL(k_qr_step<false>, grid, dim3(QT), qr_lds(x.m), s, d, k);
+    if (x.tall) hipLaunchKernelGGL(k_qr_step<true>, grid, dim3(QT), 0, s, d, k);
+  }
 }
 
 void launch_long(const DevSvd* d, const std::vector<DevSvd>& jobs, int complete, hipStream_t s) {
-  int nb = 0, m = 0;
-  for (const DevSvd& j : jobs) { nb = std::max(nb, (j.n + PB - 1) / PB); m = std::max(m, j.m); }
-  if (nb > 0) hipLaunchKernelGGL(k_svd_long, dim3(nb, (int)jobs.size()), dim3(QT), qr_lds(m), s, d, complete);
+  const Extent x(jobs);
+  const dim3 grid(x.nb, (int)jobs.size());
+  if (x.m > 0) hipLaunchKernelGGL(k_svd_long<false>, grid, dim3(QT), qr_lds(x.m), s, d, complete);
+  if (x.tall) hipLaunchKernelGGL(k_svd_long<true>, grid, dim3(QT), 0, s, d, complete);
 }
 
 }  // namespace

@@ -1,6 +1,6 @@
 """Split's decompositions at the sizes where its kernels change: panels of 16 columns, the
 Jacobi sweeps of one launch up to 32 columns and rounds of pairs of 16-column blocks above,
-wide and tall sectors, rank deficiency, and the sectors longer than the in-house limit. That
+wide and tall sectors, rank deficiency, and the sectors longer than a panel in LDS. That
 the own kernels did it, and not the rocSOLVER call that repeats a sector without convergence,
 is read from the context's counters. One left and one right sector, so that all three
 centre sectors are a x b matrices of the test's choosing."""
@@ -14,10 +14,16 @@ pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 1), (1, 40), (15, 16), (16, 15), (17, 33), (40, 40), (64, 64), (64, 70), (65, 64), (65, 65), (80, 66),
          (97, 130), (200, 190), (257, 130), (600, 610), (1024, 24), (700, 1024), (1030, 5)]
+TALL = [(1025, 1), (17, 1025), (1030, 50), (1537, 250), (256, 2049), (4096, 31)]
+
+
+def own(a, b):
+    """The sector is within the limits of the own kernels."""
+    return max(a, b) <= 1024 or (max(a, b) <= 4096 and min(a, b) <= 256)
 
 
 @pytest.mark.parametrize("rank", [None, 0.4])
-@pytest.mark.parametrize("a,b", SIZES)
+@pytest.mark.parametrize("a,b", SIZES + TALL)
 def test_split_decompositions(a, b, rank):
     L, N, st = 8, 6, 3
     T, V = hubbard(L, U=3.0)
@@ -106,7 +112,7 @@ def sides(ctx, a, b):
 
 
 @pytest.mark.parametrize("scale", ["flat", "graded"])
-@pytest.mark.parametrize("a,b", [s for s in SIZES if max(s) <= 1024])
+@pytest.mark.parametrize("a,b", SIZES + TALL)
 def test_singular_vectors_orthonormal(a, b, scale):
     # A column goes through n reflectors and some 10 n rotations, each of which rounds it by half
     # a unit in the last place of its elements: a random walk of sqrt(11 n) such steps, of 0.5 x
@@ -216,7 +222,7 @@ def test_sector_without_finite_values(a, b, bad):
 
 
 @pytest.mark.parametrize("rank", [None, 0.4])
-@pytest.mark.parametrize("a,b", SIZES)
+@pytest.mark.parametrize("a,b", SIZES + TALL + [(1025, 257), (4097, 3)])
 def test_own_kernels_converge(a, b, rank):
     print(f"case {a} x {b} rank {rank}", flush=True)
     ctx = chemps2_amd.Context(0)
@@ -224,7 +230,7 @@ def test_own_kernels_converge(a, b, rank):
         boundaries(ctx, a, b)
         ctx.s_set(graded(a, b, 1000 * a + b, rank)[1])
         ctx.split(3, 10 ** 6, moving_right=True)
-        assert ctx.split_stats() == ((3, 0, 0) if max(a, b) <= 1024 else (0, 3, 0))
+        assert ctx.split_stats() == ((3, 0, 0) if own(a, b) else (0, 3, 0))
     finally:
         ctx.close()
 
