@@ -337,7 +337,10 @@ struct Ctx : HostState {
   // (not converged)
   int64_t svd_own = 0, svd_library = 0, jacobi_retries = 0;
   int svd_max_sweeps = 0;                // CHM_SVD_MAX_SWEEPS: sweep limit of the Jacobi kernel (0: its own)
-  // Split's matrices and workspaces, kept between calls (grown as needed)
+  // Split's matrices and workspaces, grown as needed; kept between calls while they are at most
+  // SPLIT_KEEP doubles in all (a dozen allocations of some microseconds, which larger sectors do
+  // not notice)
+  static constexpr size_t SPLIT_KEEP = 16 << 20;
   struct SplitWork {
     DBuf<double> M, U, VT, S, E, W, X, J, T, F, jres;
     DBuf<int> order, rot, info, jsw;
@@ -345,6 +348,11 @@ struct Ctx : HostState {
     DBuf<DevSvd> jobs;
     void release() {
       for (DBuf<double>* b : {&M, &U, &VT, &S, &E, &W, &X, &J, &T, &F, &jres}) b->release();
+    }
+    size_t doubles() const {
+      size_t n = 0;
+      for (const DBuf<double>* b : {&M, &U, &VT, &S, &E, &W, &X, &J, &T, &F, &jres}) n += b->n;
+      return n;
     }
   } sw;
   std::vector<hipStream_t> svd_streams;

@@ -166,7 +166,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   struct Center {
     int nm, sm, im, dLt = 0, dRt = 0, cd = 0;
     bool jac = false;  // svd_batch or rocSOLVER
-    int64_t moff = 0, uoff = 0, voff = 0, soff = 0, qoff = 0, toff = 0;
+    int64_t moff = 0, uoff = 0, voff = 0, soff = 0, qoff = 0, toff = 0, woff = 0;
     std::vector<Mult> lf, rt;
   };
   std::vector<Center> cs;
@@ -194,7 +194,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     c.cd = std::min(c.dLt, c.dRt);
     cs.push_back(c);
   }
-  int64_t msz = 0, usz = 0, vsz = 0, ssz = 0, qsz = 0, tsz = 0;
+  int64_t msz = 0, usz = 0, vsz = 0, ssz = 0, qsz = 0, tsz = 0, wsz = 0;
   for (auto& c : cs) {
     if (c.cd <= 0) continue;
     // Longer sectors, those of steps near the chain's ends, have their QR panels in memory instead
@@ -209,6 +209,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
     if (c.jac) {
       c.qoff = qsz; qsz += (int64_t)c.cd * c.cd;
       c.toff = tsz; tsz += (int64_t)(c.cd + 15) / 16 * 256;
+      c.woff = wsz; wsz += (int64_t)c.dLt * c.dRt;
     }
   }
   // workspaces of svd_batch: the sorted matrices, X and J, the panels' T, floors, orders
@@ -216,7 +217,11 @@ double Ctx::split(int st, int D, bool mr, bool change) {
   DBuf<double>&M = sw.M, &U = sw.U, &VT = sw.VT, &Sg = sw.S, &E = sw.E, &Ww = sw.W, &Xw = sw.X, &Jw = sw.J, &Tw = sw.T, &Fw = sw.F;
   DBuf<int>&Iw = sw.order, &Rw = sw.rot, &info = sw.info;
   const int64_t nsec = (int64_t)cs.size();
-  Ww.alloc(std::max<int64_t>(qsz > 0 ? msz : 0, 1));
+  struct GiveBack {
+    SplitWork& w;
+    ~GiveBack() { if (w.doubles() > SPLIT_KEEP) w.release(); }
+  } give_back{sw};
+  Ww.alloc(std::max<int64_t>(wsz, 1));
   Xw.alloc(std::max<int64_t>(qsz, 1));
   Jw.alloc(std::max<int64_t>(qsz, 1));
   Tw.alloc(std::max<int64_t>(tsz, 1));
@@ -284,7 +289,7 @@ double Ctx::split(int st, int D, bool mr, bool change) {
       const auto& c = cs[q];
       if (c.cd > 0 && c.jac && sel[q]) {
         DevSvd j{};
-        j.A = M.p + c.moff; j.W = Ww.p + c.moff; j.X = Xw.p + c.qoff; j.J = Jw.p + c.qoff; j.T = Tw.p + c.toff;
+        j.A = M.p + c.moff; j.W = Ww.p + c.woff; j.X = Xw.p + c.qoff; j.J = Jw.p + c.qoff; j.T = Tw.p + c.toff;
         j.U = U.p + c.uoff; j.VT = VT.p + c.voff; j.S = Sg.p + c.soff;
         j.floor2 = Fw.p + 2 * q; j.sector = (int)q; j.perm = Iw.p + 2 * c.soff; j.src = Iw.p + 2 * c.soff + c.cd;
         j.info = info.p + q;

@@ -6,6 +6,7 @@ is read from the context's counters. One left and one right sector, so that all 
 centre sectors are a x b matrices of the test's choosing."""
 import numpy as np
 import pytest
+import torch
 
 import chemps2_amd
 from chemps2_amd.problems import hubbard, mx_table
@@ -254,5 +255,47 @@ def test_sectors_without_convergence(monkeypatch, a, b):
             assert np.abs(u.T @ u - np.eye(n)).max() <= tol
         ctx.join(3)
         assert np.linalg.norm(ctx.s_get() - x) <= tol
+    finally:
+        ctx.close()
+
+
+def test_large_workspaces_are_given_back():
+    # the matrices of a dozen sectors of up to some 1000 x 1000 take more than the 128 MB that
+    # stay with the context
+    left = [(1, 1), (2, 0), (2, 2), (3, 1), (3, 3), (4, 0), (4, 2), (5, 1)]
+    right = [(3, 1), (4, 0), (4, 2), (5, 1), (5, 3), (6, 0), (6, 2), (7, 1)]
+    d = 250
+    T, V = hubbard(8, U=3.0)
+    ctx = chemps2_amd.Context(0)
+    try:
+        ctx.set_problem(8, 0, np.zeros(8, dtype=np.int32), 8, 0, 0, mx_table(T, V, 8))
+        ctx.set_sectors_auto(10 ** 6)
+        ctx.set_sectors(3, [(n, s, 0, d) for n, s in left])
+        ctx.set_sectors(5, [(n, s, 0, d) for n, s in right])
+        ctx.set_sectors(4, [(n, s, 0, 1) for n in range(1, 8) for s in range(n % 2, 5, 2)])
+        for q in (3, 4):
+            ctx.mps_upload(q, np.ones(ctx.mps_layout_size(q)))
+        ctx.join(3)
+        # the first Split allocates the tensors of its dimensions and drops what its sectors lack
+        ctx.s_set(np.random.default_rng(3).normal(size=ctx.s_get().size))
+        ctx.split(3, 10 ** 6, moving_right=True)
+        ctx.join(3)
+        x = ctx.s_get() / np.linalg.norm(ctx.s_get())
+        ctx.s_set(x)
+        ctx.split(3, 10 ** 6, moving_right=True)
+        free = torch.cuda.mem_get_info(0)[0]
+        ctx.join(3)
+        assert np.linalg.norm(ctx.s_get() - x) <= 1e-13
+        n = sum(min(sum(d for a, t in left if 0 <= m - a <= 2 and abs(t - s) == (m - a) % 2),
+                    sum(d for a, t in right if 0 <= a - m <= 2 and abs(t - s) == (a - m) % 2)) ** 2
+                for m in range(1, 8) for s in range(m % 2, 5, 2))
+        print(f"sectors of {n} elements in all", flush=True)
+        assert 6 * 8 * n > 128 << 20
+        tensors = 8 * sum(ctx.mps_layout_size(q) for q in (3, 4))
+        ctx.close()
+        held = torch.cuda.mem_get_info(0)[0] - free
+        print(f"held {held >> 20} MiB, tensors {tensors >> 20} MiB, object {x.nbytes >> 20} MiB", flush=True)
+        # the tensors, the object and the join's lists besides, and the math library's own
+        assert held <= tensors + 4 * x.nbytes + (128 << 20)
     finally:
         ctx.close()
