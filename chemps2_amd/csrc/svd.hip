@@ -361,13 +361,14 @@ struct Rot {
   double s, h;
 };
 __device__ __forceinline__ Rot rotation(double al, double be, double ga, double tol2, double fl) {
-  const double d = be - al, r = __builtin_amdgcn_sqrt(fma(d, d, 4.0 * ga * ga));
-  const double t = (d >= 0.0 ? 2.0 : -2.0) * ga * __builtin_amdgcn_rcp(fabs(d) + r);
-  const double c = __builtin_amdgcn_rsq(fma(t, t, 1.0)), h = t * c * __builtin_amdgcn_rcp(1.0 + c);
+  // cos of twice the angle is |d| / |(d, 2 ga)|; q = cos^2 of the angle
+  const double d = be - al, ri = __builtin_amdgcn_rsq(fma(d, d, 4.0 * ga * ga)), q = fma(0.5 * fabs(d), ri, 0.5);
+  const double ci = __builtin_amdgcn_rsq(q), c1 = fma(q, ci, 1.0);
+  const double h = (d >= 0.0 ? ga : -ga) * ri * ci * __builtin_amdgcn_rcp(c1);
   // 1 / (1 + h^2) = (1 + cos) / 2
-  const double q = fma(0.5, c, 0.5), e = fma(-fma(h, h, 1.0), q, 1.0);
+  const double w = 0.5 * c1, e = fma(-fma(h, h, 1.0), w, 1.0);
   const bool on = al > fl && be > fl && ga * ga > tol2 * (al * be);
-  return on ? Rot{2.0 * h * fma(q, fma(e, e, e), q), h} : Rot{0.0, 0.0};
+  return on ? Rot{2.0 * h * fma(w, fma(e, e, e), w), h} : Rot{0.0, 0.0};
 }
 // (u, v) <- (c u - s v, s u + c v), with c = 1 - s h: what rounding and an s that is not quite
 // sin take from the columns' orthogonality is smaller than with c by a factor of s, and not of
