@@ -12,6 +12,7 @@
 #include "../../include/chemps2_amd.h"
 #include "context.hpp"
 #include "parallel.hpp"
+#include "segments.hpp"
 
 namespace chm {
 
@@ -1077,31 +1078,11 @@ void Ctx::prepare(int st) {
     });
   }
   const int64_t nblk = (int64_t)bwork.size();
-  std::vector<int> bseg(nblk, 1);
+  std::vector<int> bseg;
   {
-    // chunks of the blocks that fit a wavefront's 32 x 32, and of the others (per 64 x 64 tile)
-    int64_t wsmall = 0, wlarge = 0;
-    auto small = [&](int64_t bi) { return dLof(chain[bq[bi]]->out) <= 32 && dRof(chain[bq[bi]]->out) <= 32; };
-    for (int64_t bi = 0; bi < nblk; bi++) {
-      const int k = chain[bq[bi]]->out;
-      (small(bi) ? wsmall : wlarge) += bwork[bi] * ((dLof(k) + 63) / 64) * ((dRof(k) + 63) / 64);
-    }
-    // segments of ws / wl chunks; returns the partial sums they need
-    auto cut = [&](int64_t ws, int64_t wl) {
-      int64_t part = 0;
-      for (int64_t bi = 0; bi < nblk; bi++) {
-        bseg[bi] = (int)std::max<int64_t>(1, std::min<int64_t>(bwork[bi] / std::max<int64_t>(std::max(1, tile_seg_min), small(bi) ? ws : wl), 64));
-        if (bseg[bi] > 1) part += (int64_t)bseg[bi] * dLof(chain[bq[bi]]->out) * dRof(chain[bq[bi]]->out);
-      }
-      return part;
-    };
-    // A long list gets enough segments of either kind to fill the device (a wavefront takes one
-    // of the small blocks': four times as many; 11.3 -> 10.6 ms a product at the L = 32, D = 2000
-    // middle site), unless their partial sums would near the static scratch of
-    // chm_heff_apply_noalloc; a short list one target over both.
-    const int64_t seg = std::max(1, tile_segments);
-    if (!share || cut(wsmall / (2 * seg), wlarge / seg) + bpart_need > ((int64_t)28 << 20))
-      cut((wsmall + wlarge) / seg, (wsmall + wlarge) / seg);
+    std::vector<SegBlock> blocks(nblk);
+    for (int64_t bi = 0; bi < nblk; bi++) blocks[bi] = {bwork[bi], dLof(chain[bq[bi]]->out), dRof(chain[bq[bi]]->out)};
+    choose_segments(blocks, share, std::max(1, tile_segments), std::max(1, tile_seg_min), bpart_need, cpart_need, bseg);
   }
   // Segment boundaries (about equal chunk counts) and whether a segment holds an axpy
   // product, per block on the host threads; then the tiles per batch in TILE2_RANGES ranges of

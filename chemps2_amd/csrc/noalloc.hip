@@ -13,11 +13,11 @@
 
 #include "../../include/chemps2_amd.h"
 #include "context.hpp"
+#include "segments.hpp"
 
 namespace {
 
-// 32 Mi doubles (256 MiB) of partial sums
-constexpr int64_t kScratchDoubles = int64_t(1) << 25;
+constexpr int64_t kScratchDoubles = chm::NOALLOC_DOUBLES;
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
 constexpr int kMaxDevices = 64;
