@@ -465,6 +465,13 @@ inline int tile_bucket(int mrem, int nrem) {
   if (mrem <= 16) return 6;
   return ((mrem + 15) / 16 * ((nrem + 15) / 16) + 3) / 4;
 }
+// the bucket of a workgroup's tile (c = 1..4) at any size: k_tiles_stream1 has 64-bit offsets
+inline int tile_bucket_wide(int mrem, int nrem) { return ((mrem + 15) / 16 * ((nrem + 15) / 16) + 3) / 4; }
+// The wavefront tiles, k_tiles_fit and k_strips take a block's elements by 32-bit byte offsets off a
+// uniform base (one register and one instruction an address; 64-bit offsets cost 1 % of a product
+// at the chain's end). Where a block may have TILE_WIDE_MIN elements, k_tiles_stream1 and
+// k_tiles_mfma do all tiles.
+constexpr int64_t TILE_WIDE_MIN = (int64_t)1 << 28;
 bool strip_kernel_setup();  // false: the device refuses the widest bucket's LDS
 void launch_strips(const DevXGroup* groups, int ngroups, const DevStripW* ws, int bucket, const double* xbase,
                    hipStream_t s);

@@ -896,11 +896,13 @@ void Ctx::prepare(int st) {
   tb1.assign(1, 0);
   tb2.assign(1, 0);
   // tiles of 64 x 64 by bucket, or (wave_tiles) of 32 x 32, all on wavefronts
-  const int ts1 = wave_tiles ? 32 : 64;
+  tiles_wide = site_dmax * site_dmax >= tile_wide_min;
+  const bool wave32 = wave_tiles && !tiles_wide;
+  const int ts1 = wave32 ? 32 : 64;
   auto each_tile = [&](const WDim& w, auto&& f) {
     for (int m0 = 0; m0 < w.rows; m0 += ts1)
       for (int n0 = 0; n0 < w.cols; n0 += ts1)
-        f(m0, n0, wave_tiles ? 0 : tile_bucket(std::min(64, w.rows - m0), std::min(64, w.cols - n0)));
+        f(m0, n0, wave32 ? 0 : (tiles_wide ? tile_bucket_wide : tile_bucket)(std::min(64, w.rows - m0), std::min(64, w.cols - n0)));
   };
   // Per batch: the two-operand terms grouped by input block (a counting sort, stable), the
   // distinct W of every group by a hash of the operator block, then W offsets and the
@@ -919,7 +921,7 @@ void Ctx::prepare(int st) {
     std::array<int32_t, STRIP_BUCKETS> xg{};
   };
   // A W goes to k_strips in a long list when its inner dimension fits, else to the tiles.
-  const bool use_strips = share && strips_ok;
+  const bool use_strips = share && strips_ok && !tiles_wide;
   // fewer strips per group in the shorter lists, so that the groups still fill the device
   const int strip_group = (int)std::max<int64_t>(8, std::min<int64_t>(STRIP_GROUP, ntwo / 16384));
   auto w_strip = [&](const Term& t, bool rf) { return use_strips && (rf ? dRof(t.in) : dLof(t.in)) <= STRIP_MAXK; };
@@ -1115,12 +1117,12 @@ void Ctx::prepare(int st) {
   // the tiles of an output block (segment): 64 x 64, those of at most 32 x 32 on wavefronts; or
   // (wave_tiles) 32 x 32 on wavefronts unless the segment has an axpy
   auto each_tile2 = [&](int dL, int dR, bool ax, auto&& f) {
-    const bool q32 = wave_tiles && !ax;
+    const bool q32 = wave32 && !ax;
     const int st = q32 ? 32 : 64;
     for (int m0 = 0; m0 < dL; m0 += st)
       for (int n0 = 0; n0 < dR; n0 += st) {
         const int mr = std::min(st, dL - m0), nr = std::min(st, dR - n0);
-        f(m0, n0, mr <= 32 && nr <= 32 ? (share ? wave_shape(mr, nr) : 3) : TILE2_RANGES - 1);
+        f(m0, n0, mr <= 32 && nr <= 32 && !tiles_wide ? (share ? wave_shape(mr, nr) : 3) : TILE2_RANGES - 1);
       }
   };
   std::vector<std::array<int64_t, TILE2_RANGES>> tile2(nblk);  // first tile of a block in every range
@@ -1409,7 +1411,7 @@ void Ctx::apply_with(const double* xp, double* yp, double* bp, double* cp, doubl
       launch_tiles_stream1(tiles1.p + tb1[i], tb1[i + 1] - tb1[i], c, xp, stream);
     }
     const int* r = tb2.data() + TILE2_RANGES * b;
-    launch_tiles(tiles2.p + r[4], ops2.p, r[5] - r[4], xp, yp, stream, tiles_kernel, cp);
+    launch_tiles(tiles2.p + r[4], ops2.p, r[5] - r[4], xp, yp, stream, tiles_wide ? std::min(tiles_kernel, 1) : tiles_kernel, cp);
     for (int q = 3; q >= 0; q--) launch_tiles_wave2(tiles2.p + r[q], ops2.p, r[q + 1] - r[q], q, xp, yp, stream, cp);
   }
   launch_chain_reduce(treds.p, ntreds, cp, yp, stream);  // segments of split output blocks
@@ -1573,17 +1575,19 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
   // output block of every term; phase-1 counts per segment (k_ops items or GEMM tiles)
   struct P1 {
     int64_t ops = 0, items = 0, w = 0;
+    int dmax = 0;  // the largest dimension of its blocks
     std::array<int64_t, TILE_BUCKETS> tiles{};
   };
-  auto each_tile1 = [](int m, int nn, auto&& f) {  // 64 x 64 tiles by bucket (tile_bucket)
+  bool wide = false;  // no tiles on wavefronts and no k_tiles_fit: a block of tile_wide_min elements
+  auto each_tile1 = [&](int m, int nn, auto&& f) {  // 64 x 64 tiles by bucket (tile_bucket)
     for (int m0 = 0; m0 < m; m0 += 64)
       for (int n0 = 0; n0 < nn; n0 += 64) {
         const int mr = std::min(64, m - m0), nr = std::min(64, nn - n0);
-        f(m0, n0, mr, nr, tile_bucket(mr, nr));
+        f(m0, n0, mr, nr, wide ? tile_bucket_wide(mr, nr) : tile_bucket(mr, nr));
       }
   };
   std::vector<P1> p1(nseg + 1);
-  parallel_for(nseg, nthr, [&](int64_t s, int) {
+  auto count1 = [&](int64_t s, int) {
     P1 c;
     int last = -1;  // consecutive terms mostly write the same block
     for (size_t j = 0; j < segs[s].terms.size(); j++) {
@@ -1595,6 +1599,7 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
       if (qq < 0) throw Error{ERR_STATE, "operator update term writes outside the new tensors"};
       qof[s0[s] + j] = qq;
       seg_of[s0[s] + j] = (int)s;
+      c.dmax = std::max({c.dmax, u.m, u.n, u.kind == 2 ? 0 : u.k1, u.kind == 1 ? u.k2 : 0});
       if (u.kind != 1) continue;
       c.ops++;
       if (ops_on && small_gemm(u.m, u.k2, u.k1, u.ta, u.lda, u.tb, u.ldb)) c.items++;
@@ -1602,7 +1607,14 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
       c.w += ((int64_t)u.m * u.k2 + 7) / 8 * 8;
     }
     p1[s + 1] = c;
-  });
+  };
+  parallel_for(nseg, nthr, count1);
+  int64_t dmax = 0;
+  for (int64_t s = 0; s < nseg; s++) dmax = std::max<int64_t>(dmax, p1[s + 1].dmax);
+  if (!wide && dmax * dmax >= tile_wide_min) {
+    wide = true;
+    parallel_for(nseg, nthr, count1);
+  }
   for (int64_t s = 0; s < nseg; s++) {
     p1[s + 1].ops += p1[s].ops; p1[s + 1].items += p1[s].items; p1[s + 1].w += p1[s].w;
     for (int b = 0; b < TILE_BUCKETS; b++) p1[s + 1].tiles[b] += p1[s].tiles[b];
@@ -1676,7 +1688,7 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
         i2start[q + 1] = ni;
         p2start[q + 1] = ni > 1 ? ni * (int64_t)m * nn : 0;
       } else {
-        each_tile1(m, nn, [&](int, int, int mr, int nr, int) { (mr <= 32 && nr <= 32 ? tw2start : t2start)[q + 1]++; });
+        each_tile1(m, nn, [&](int, int, int mr, int nr, int) { (mr <= 32 && nr <= 32 && !wide ? tw2start : t2start)[q + 1]++; });
       }
     }
   });
@@ -1794,7 +1806,7 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
           tl.C = C; tl.ldc = m; tl.m0 = m0; tl.n0 = n0; tl.m = m; tl.n = nn;
           tl.op0 = (int)qstart[q]; tl.nop = (int)(qstart[q + 1] - qstart[q]);
           tl.flags = axpy ? 0 : TILE_NO_AXPY;
-          t2[mr <= 32 && nr <= 32 ? itw++ : it++] = tl;
+          t2[mr <= 32 && nr <= 32 && !wide ? itw++ : it++] = tl;
         });
       }
     }
@@ -1821,7 +1833,7 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
     launch_tiles_stream1(u_dt1.p + b1[b], (int)(b1[b + 1] - b1[b]), b, nullptr, stream);
   launch_ops(u_it1.p, (int)ni1, u_d1.p, P, stream);
   launch_tiles_wave2(u_dt2.p, u_d2.p, (int)ntw2, 3, nullptr, nullptr, stream);
-  launch_tiles(u_dt2.p + ntw2, u_d2.p, (int)(nt2 - ntw2), nullptr, nullptr, stream, tiles_kernel);
+  launch_tiles(u_dt2.p + ntw2, u_d2.p, (int)(nt2 - ntw2), nullptr, nullptr, stream, wide ? std::min(tiles_kernel, 1) : tiles_kernel);
   launch_ops(u_it2.p, (int)ni2, u_d2.p, P, stream);
   launch_part_reduce(u_rd.p, (int)nred, u_part.p, stream);
   hip_check(hipGetLastError(), "update kernels");
@@ -2602,6 +2614,7 @@ int chm_ctx_create(int device, chm_ctx** out) {
   if (const char* e = std::getenv("CHM_CHAIN_ITEM_TERMS")) ctx->c.chain_item_terms = std::max(1, std::atoi(e));
   if (const char* e = std::getenv("CHM_CHAIN_GROUP_TERMS")) ctx->c.chain_group_terms = std::max(1, std::atoi(e));
   if (const char* e = std::getenv("CHM_SVD_GESVDJ")) ctx->c.svd_large_gesvdj = std::atoi(e) != 0;
+  if (const char* e = std::getenv("CHM_TILE_WIDE_MIN")) ctx->c.tile_wide_min = std::max(0LL, std::atoll(e));
   if (const char* e = std::getenv("CHM_TILE_SHARE_MIN")) ctx->c.tile_share_min = std::atoll(e);
   if (const char* e = std::getenv("CHM_SVD_MAX_SWEEPS")) ctx->c.svd_max_sweeps = std::max(0, std::atoi(e));
   if (const char* e = std::getenv("CHM_TILE_W_CAP")) ctx->c.tile_w_cap = std::max(1LL, std::atoll(e));

@@ -158,6 +158,8 @@ struct Ctx : HostState {
   int tile_seg_min = 64;      // CHM_TILE_SEG_MIN: fewest 16-deep k chunks per segment
   bool wave_tiles = false;    // CHM_WAVE_TILES=1: every tile 32 x 32 on one wavefront (no LDS sharing)
   int64_t tile_share_min = 65536;  // CHM_TILE_SHARE_MIN: two-operand terms from which W are shared
+  int64_t tile_wide_min = TILE_WIDE_MIN;  // CHM_TILE_WIDE_MIN: block elements from which tiles use 64-bit offsets
+  bool tiles_wide = false;         // the prepared site's tiles do
   int64_t tile_w_cap = 0;  // doubles of W scratch per batch (CHM_TILE_W_CAP; 0: a quarter of free memory)
   DBuf<DevGemmOp> ops2;
   int ntiles1 = 0, ntiles2 = 0;
@@ -251,7 +253,9 @@ struct Ctx : HostState {
   bool svd_large_gesvdj = true;      // CHM_SVD_GESVDJ=0: large Split sectors by rocsolver_dgesvd instead of dgesvdj
   int chain_item_terms = CHAIN_ITEM_TERMS;    // CHM_CHAIN_ITEM_TERMS
   int chain_group_terms = CHAIN_GROUP_TERMS;  // CHM_CHAIN_GROUP_TERMS
-  int tiles_kernel = 2;  // CHM_TILES_MFMA: grouped GEMM tiles (Heff phase 2, updates) in 2 k_tiles_fit, 1 k_tiles_mfma, 0 k_tiles
+  // CHM_TILES_MFMA: the grouped GEMM tiles that are not on wavefronts in 2 k_tiles_fit, 1
+  // k_tiles_mfma, 0 k_tiles
+  int tiles_kernel = 2;
   int cblocks_m_offs[CHAIN_MFMA_NT + 1] = {};
   DBuf<DevCBlock> cblocks;
   DBuf<DevCGroup> cgroups;

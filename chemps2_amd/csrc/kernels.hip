@@ -353,7 +353,7 @@ __device__ __forceinline__ void tiles_fit_body(const DevTile& t, const DevGemmOp
     if (op.tb == 0) { kb = tid & 15; c = (tid >> 4) + 16 * q; } else { c = tid & 63; kb = (tid >> 6) + 4 * q; }
   };
   // raw global (not flat) loads of chunk (op, kc), with 32-bit byte offsets off a uniform base
-  // (a block holds fewer than 2^28 elements); a lane outside the block reads the block's first
+  // (a block holds fewer than TILE_WIDE_MIN elements); a lane outside it reads its first
   // element: put applies the masks and alpha, so nothing here waits for the loads
   auto fetch = [&](const FitOp& op, int kc, double (&ra)[4], double (&rb)[4]) {
     gbyte* A = (gbyte*)op.A;
@@ -644,7 +644,7 @@ struct TwOp {  // one product on one tile, pointers resolved
 // The helpers below work on an MS x NS grid of 16 x 16 sub-tiles per wavefront (2 x 2:
 // tiles of at most 32 x 32; 4 x 1 and 1 x 4: the thin tiles of at most 64 x 16 and 16 x 64).
 // raw loads of chunk (f, k0); 32-bit byte offsets (an operator block or x holds fewer
-// than 2^28 elements), so that the loads take the uniform base from scalar registers
+// than TILE_WIDE_MIN elements), so that the loads take the uniform base from scalar registers
 template <int MS, int NS>
 __device__ __forceinline__ void tw_fetch(const TwOp& f, int k0, int lr, int lg, double (&pa)[4][MS], double (&pb)[4][NS]) {
   gbyte* A = (gbyte*)f.A;
@@ -871,7 +871,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(3, 8))) void
 // Phase 1 of a long list with the input block in LDS: a workgroup loads its group's columns
 // (or rows) of x once, zero-padded; its wavefronts then walk the group's W, 16 rows (columns)
 // of the operator at a time, without barriers: a strip's operator elements come straight
-// into registers, the next strip's in flight while this one computes. Roles in the MFMA
+// into registers (32-bit offsets as in k_tiles_fit), the next strip's in flight while this one computes. Roles in the MFMA
 // are chosen so that W is stored along its columns. Before, every W was a tile of its own
 // that staged both operands (k_tiles_stream1, k_tiles_wave1): 5.0 ms for the 1.23 M W (42 GF,
 // 4.4 GB written) of the L = 32, D = 2000 middle site, 3.7 ms here.

@@ -16,8 +16,8 @@ LEFT = [(2, 0), (2, 2), (3, 1), (3, 3), (4, 0), (4, 2)]   # (N, 2S) at the left 
 RIGHT = [(4, 0), (4, 2), (5, 1), (5, 3), (6, 0), (6, 2)]
 
 
-def product(dims, x, share, w_cap=None):
-    env = {"CHM_TILE_SHARE_MIN": str(share), "CHM_EXPLICIT_MAX": "1"}
+def product(dims, x, share, w_cap=None, **more):
+    env = {"CHM_TILE_SHARE_MIN": str(share), "CHM_EXPLICIT_MAX": "1", **more}
     if w_cap:
         env["CHM_TILE_W_CAP"] = str(w_cap)
     old = {k: os.environ.get(k) for k in env}
@@ -58,3 +58,14 @@ def test_long_lists_equal_short_lists(dims):
     # thousand terms per element: errors of 2^-53 each, as a random walk
     assert np.abs(y1 - y0).max() <= 64 * 2.0 ** -53 * np.sqrt(s0["chain_terms"]) * np.abs(y0).max()
     assert np.abs(y2 - y0).max() <= 64 * 2.0 ** -53 * np.sqrt(s0["chain_terms"]) * np.abs(y0).max()
+
+
+@pytest.mark.parametrize("share", [1, 10 ** 9])
+@pytest.mark.parametrize("dims", [(1, 2, 3), (31, 5, 33), (65, 80, 63)])
+def test_tiles_for_blocks_of_any_size(dims, share):
+    # with 64-bit offsets, as for blocks of 2^28 elements and more
+    print(f"case dims {dims} share {share}", flush=True)
+    x, y0, s0 = product(dims, None, 10 ** 9)
+    _, y1, s1 = product(dims, x, share, CHM_TILE_WIDE_MIN="0")
+    assert s1["chain_terms"] == s0["chain_terms"] > 0
+    assert np.abs(y1 - y0).max() <= 64 * 2.0 ** -53 * np.sqrt(s0["chain_terms"]) * np.abs(y0).max()

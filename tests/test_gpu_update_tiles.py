@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import chemps2_amd
-from chemps2_amd.problems import random_abinitio
+from chemps2_amd.problems import mx_table, random_abinitio
 from plancheck import oracle_tensors
 
 pytestmark = pytest.mark.gpu
@@ -74,9 +74,15 @@ def update(shapes, mr, dims, uv, scalars):
         c.close()
 
 
+@pytest.mark.parametrize("sizes", [(3, 17, 5), (33, 48, 16), (65, 5, 97)])
+def test_update_in_tiles_for_blocks_of_any_size(monkeypatch, shapes, sizes):
+    monkeypatch.setenv("CHM_TILE_WIDE_MIN", "0")
+    test_update_of_rank_one_blocks(shapes, sizes, True)
+
+
 @pytest.mark.parametrize("mr", [True, False])
 @pytest.mark.parametrize("sizes", [(1, 2, 17), (15, 16, 33), (31, 32, 9), (33, 48, 16), (63, 64, 31), (65, 5, 97), (128, 64, 129)])
-def test_update_of_rank_one_blocks(shapes, mr, sizes):
+def test_update_of_rank_one_blocks(shapes, sizes, mr):
     print(f"case sizes {sizes} moving_right {mr}", flush=True)
     rng = np.random.default_rng(2)
     keys = [("l", n, s) for n, s in LEFT] + [("r", n, s) for n, s in RIGHT]
@@ -97,3 +103,40 @@ def test_update_of_rank_one_blocks(shapes, mr, sizes):
         assert np.abs(g - spread(s, bl, side)).max(initial=0) <= 3e-13 * scale
         seen += g.size > 0
     assert seen > 30
+
+
+@pytest.mark.parametrize("rows,cols", [(128, 40), (80, 24)])
+def test_blocks_of_more_than_four_gigabytes(rows, cols):
+    # Join of a left block of more than 2^29 elements, whose last columns alone are not zero: byte
+    # offsets beyond 32 bits, in tiles of 64 x 40, 64 x 24 and 16 x 24
+    mid = 2 ** 29 // rows + 48
+    print(f"case {rows} x {mid} x {cols}", flush=True)
+    c = chemps2_amd.Context(0)
+    try:
+        irr, T, V = random_abinitio(L, 4, group=G)
+        c.set_problem(L, G, irr, 8, 0, 0, mx_table(T, V, 8))
+        c.set_sectors(3, [(2, 0, 0, rows)])
+        c.set_sectors(4, [(3, 1, 0, mid)])
+        c.set_sectors(5, [(4, 0, 0, cols)])
+        rng = np.random.default_rng(rows)
+        a, b = rng.normal(size=(rows, 48)), rng.normal(size=(48, cols))
+        assert c.mps_layout_size(3) == rows * mid and c.mps_layout_size(4) == mid * cols
+        left = np.zeros(rows * mid)
+        left[-rows * 48:] = a.ravel("F")
+        c.mps_upload(3, left)
+        del left
+        right = np.zeros((cols, mid))
+        right[:, -48:] = b.T
+        c.mps_upload(4, right.ravel())
+        del right
+        c.join(3)
+        got = c.s_get()
+        ref = a @ b
+        blocks = [g.reshape(cols, rows).T for g in got.reshape(-1, rows * cols) if np.abs(g).max() > 0]
+        assert blocks
+        for g in blocks:  # each a recoupling factor times the product; 48 terms a sum
+            f = np.vdot(g, ref) / np.vdot(ref, ref)
+            assert abs(f) > 0.1
+            assert np.abs(g - f * ref).max() <= 48 * 2.0 ** -52 * abs(f) * np.abs(ref).max()
+    finally:
+        c.close()
