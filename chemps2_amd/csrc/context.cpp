@@ -1578,7 +1578,8 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
     int dmax = 0;  // the largest dimension of its blocks
     std::array<int64_t, TILE_BUCKETS> tiles{};
   };
-  bool wide = false;  // no tiles on wavefronts and no k_tiles_fit: a block of tile_wide_min elements
+  // no tiles on wavefronts and no k_tiles_fit: asked for, or a block of tile_wide_min elements
+  bool wide = tiles_kernel != 2;
   auto each_tile1 = [&](int m, int nn, auto&& f) {  // 64 x 64 tiles by bucket (tile_bucket)
     for (int m0 = 0; m0 < m; m0 += 64)
       for (int n0 = 0; n0 < nn; n0 += 64) {
@@ -1833,15 +1834,15 @@ void Ctx::run_terms(const std::vector<USeg>& segs, const std::vector<std::pair<R
     launch_tiles_stream1(u_dt1.p + b1[b], (int)(b1[b + 1] - b1[b]), b, nullptr, stream);
   launch_ops(u_it1.p, (int)ni1, u_d1.p, P, stream);
   launch_tiles_wave2(u_dt2.p, u_d2.p, (int)ntw2, 3, nullptr, nullptr, stream);
-  launch_tiles(u_dt2.p + ntw2, u_d2.p, (int)(nt2 - ntw2), nullptr, nullptr, stream, wide ? std::min(tiles_kernel, 1) : tiles_kernel);
+  launch_tiles(u_dt2.p + ntw2, u_d2.p, (int)(nt2 - ntw2), nullptr, nullptr, stream, wide ? std::min(tiles_kernel, 1) : 2);
   launch_ops(u_it2.p, (int)ni2, u_d2.p, P, stream);
   launch_part_reduce(u_rd.p, (int)nred, u_part.p, stream);
   hip_check(hipGetLastError(), "update kernels");
   hip_check(hipStreamSynchronize(stream), "update");
   if (verbose)
-    std::fprintf(stderr, "    terms %lld: lists %.3f s (map %.3f, sort %.3f, counts %.3f, fill %.3f), upload %.3f s, kernels %.3f s (%lld + %lld tiles, %lld + %lld small items)\n",
+    std::fprintf(stderr, "    terms %lld: lists %.3f s (map %.3f, sort %.3f, counts %.3f, fill %.3f), upload %.3f s, kernels %.3f s (%lld + %lld tiles, %lld of the output's on wavefronts, %lld + %lld small items)\n",
                  (long long)n, t_lists - t_begin, t_map - t_begin, t_sort - t_map, t_counts - t_sort, t_lists - t_counts,
-                 t_up - t_lists, now_s() - t_up, (long long)nt1, (long long)nt2, (long long)ni1, (long long)ni2);
+                 t_up - t_lists, now_s() - t_up, (long long)nt1, (long long)nt2, (long long)ntw2, (long long)ni1, (long long)ni2);
 }
 
 // DMRG::updateMovingRight/Left (DMRGoperators.cpp:243-907) for slot `index`.

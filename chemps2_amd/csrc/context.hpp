@@ -254,7 +254,7 @@ struct Ctx : HostState {
   int chain_item_terms = CHAIN_ITEM_TERMS;    // CHM_CHAIN_ITEM_TERMS
   int chain_group_terms = CHAIN_GROUP_TERMS;  // CHM_CHAIN_GROUP_TERMS
   // CHM_TILES_MFMA: the grouped GEMM tiles that are not on wavefronts in 2 k_tiles_fit, 1
-  // k_tiles_mfma, 0 k_tiles
+  // k_tiles_mfma, 0 k_tiles; with 1 and 0 the updates' output tiles are never on wavefronts
   int tiles_kernel = 2;
   int cblocks_m_offs[CHAIN_MFMA_NT + 1] = {};
   DBuf<DevCBlock> cblocks;

@@ -1,6 +1,8 @@
 """Operator updates at block dimensions around the edges of the 16 x 16, 32 x 32 and 64 x 64
 tiles. Every block is a scalar times u v^T with a unit vector for each sector, so an update of
 any dimensions is the update of the scalars (all dimensions 1), times the same u v^T."""
+import re
+
 import numpy as np
 import pytest
 
@@ -74,10 +76,17 @@ def update(shapes, mr, dims, uv, scalars):
         c.close()
 
 
+@pytest.mark.parametrize("env", [None, ("CHM_TILE_WIDE_MIN", "0"), ("CHM_TILES_MFMA", "1"), ("CHM_TILES_MFMA", "0")])
 @pytest.mark.parametrize("sizes", [(3, 17, 5), (33, 48, 16), (65, 5, 97)])
-def test_update_in_tiles_for_blocks_of_any_size(monkeypatch, shapes, sizes):
-    monkeypatch.setenv("CHM_TILE_WIDE_MIN", "0")
+def test_update_in_workgroup_tiles(monkeypatch, capfd, shapes, sizes, env):
+    # the tiles for blocks of any number of elements, and the older kernels on request, take all of
+    # the output; by default the blocks of at most 32 x 32 are on wavefronts
+    monkeypatch.setenv("CHM_VERBOSE", "1")
+    if env:
+        monkeypatch.setenv(*env)
     test_update_of_rank_one_blocks(shapes, sizes, True)
+    waves = [int(n) for n in re.findall(r"(\d+) of the output's on wavefronts", capfd.readouterr().err)]
+    assert waves and (not any(waves) if env else all(waves))
 
 
 @pytest.mark.parametrize("mr", [True, False])
