@@ -27,7 +27,9 @@ Workload (the metric's configuration): random ab-initio Hamiltonian with D2h sym
    the host cores: its first left-sweep steps from the same checkpoint (the same
    Heff matrices), Davidson products x F_H over the Davidson time of those steps.
 
-One JSON line goes to stdout; progress goes to stderr.
+One JSON line of less than 2000 characters goes to stdout (a reader of the end of the output gets
+it whole); what does not fit (per-site energies and products, plan and phase figures) goes to
+the file of --detail; progress goes to stderr.
 """
 import argparse
 import json
@@ -80,6 +82,24 @@ def roofline_record(F_H, B_H, ms, traffic, traffic_source):
         "traffic_over_B_H": round(traffic / B_H, 2) if traffic else None,
         "traffic_source": traffic_source,
     }
+
+
+def summary(out):
+    """The printed record: out without what belongs in the detail file."""
+    line = {k: v for k, v in out.items()
+            if k not in ("roofline", "cpu_baseline", "warm_up", "site_bench", "sweep", "n2_ccpvdz_published_point")}
+    r, cpu, sb, n2 = (out.get(k) for k in ("roofline", "cpu_baseline", "site_bench", "n2_ccpvdz_published_point"))
+    if r:
+        line["roofline"] = {k: r[k] for k in ("bound", "achieved", "peak", "unit", "frac", "traffic", "traffic_over_B_H")}
+    if cpu:
+        line["cpu_baseline"] = {k: cpu[k] for k in ("value", "unit", "cores", "kind")}
+    if sb:
+        line["site_bench"] = {k: sb[k] for k in ("site", "V", "ms_kernels", "tflops")}
+    line["sweep"] = {name: {k: s[k] for k in ("seconds", "total_min_energy", "heff_tflops_sweep_average",
+                                              "delta_E_vs_fp64") if k in s} for name, s in out["sweep"].items()}
+    if n2:
+        line["n2_ccpvdz"] = {k: n2[k] for k in ("seconds_per_sweep", "energy", "speedup_vs_published")}
+    return line
 
 
 def traffic_from(fetch_csv, write_csv, steps, out_name):
@@ -372,6 +392,8 @@ def main():
     ap.add_argument("--traffic-from", nargs=2, metavar=("FETCH_CSV", "WRITE_CSV"),
                     help="write profiles/" + "heff_site15_L32_D2000_traffic.json from the counter_collection.csv "
                     "of two --site-from runs under rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE (--steps as in those runs)")
+    ap.add_argument("--detail", metavar="JSON", default=os.path.join(tempfile.gettempdir(), "chm_bench_detail.json"),
+                    help="file of the whole record")
     args = ap.parse_args()
     if args.traffic_from:
         print(json.dumps(traffic_from(args.traffic_from[0], args.traffic_from[1], args.steps,
@@ -471,7 +493,13 @@ def main():
         "sweep": sweeps,
         "n2_ccpvdz_published_point": n2,
     }
-    print(json.dumps(out), flush=True)
+    try:
+        with open(args.detail, "w") as f:
+            json.dump(out, f, indent=1)
+        log(f"whole record: {args.detail}")
+    except OSError as e:
+        log(f"whole record not written: {e}")
+    print(json.dumps(summary(out)), flush=True)
 
 
 if __name__ == "__main__":

@@ -78,3 +78,40 @@ def test_roofline_record_hbm_bound():
     assert r["achieved"] == 1.0
     assert r["frac"] == 0.125
     assert r["traffic_over_B_H"] is None
+
+
+def test_printed_record_is_short():
+    # of a run's size: 60 sites in each of three forms
+    sweep = {"seconds": 1234.567, "presolve_seconds": 1.234, "total_min_energy": -45.762898269479706,
+             "heff_applications": 12345, "heff_applications_hi_only": 12345, "heff_flops": 1.5437882058412345e17,
+             "heff_device_seconds": 1234.5678, "heff_tflops_sweep_average": 17.1234,
+             "phase_seconds": {k: 123.456 for k in ("join", "prepare", "davidson", "split", "update", "total")},
+             "sites": [{"site": q, "energy": -45.762898269479706, "products": 12, "heff_ms": 123.456,
+                        "F_H": 154378820584.0} for q in range(60)],
+             "delta_E_vs_fp64": 2.5437429940211587e-12, "speedup_vs_fp64": 0.926}
+    sb = {"site": 15, "V": 186316, "F_H": 1.234e11, "B_H": 1.234e9, "ms_kernels": 10.1234, "ms_per_call": 10.1234,
+          "tflops": 17.1234, "kernel_ms": [1.0, 2.0, 3.0], "plan_stats": {str(q): 10 ** 9 for q in range(16)}}
+    out = {
+        "metric": "Heff\u00b7x TFLOP/s + Davidson sweep time at L=32 D=2000; |\u0394E| vs FP64 \u22641e-8 Ha",
+        "value": 17.1234, "unit": "TFLOP/s", "n_gpus": 1, "steps": 12345, "warmup": 5, "ms_per_step": 10.1234,
+        "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f64", "data": "synthetic",
+        "config": {"workload": "w" * 160, "L": 32, "D": 2000, "davidson_rtol": 1e-5, "sweep_seconds_fp64": 1234.567},
+        "roofline": bench.roofline_record(1.2345678901234e11, 1.2345678901234e9, 10.1234, 54512345678.9, "profiles/" + "t" * 40),
+        "cpu_baseline": {"value": 0.123456789012345, "unit": "TFLOP/s", "cores": 256, "kind": "reference",
+                         "sample": "s" * 500, "seconds_per_step": [1.0] * 30, "presolve_seconds": 1.0},
+        "warm_up": {"seconds": 100.0}, "site_bench": sb,
+        "sweep": {"fp64": sweep, "mixed": sweep, "mixed+learned": sweep},
+        "n2_ccpvdz_published_point": {"seconds_per_sweep": 15.184, "energy": -109.28215523999137, "warm_up_seconds": 18.06,
+                                      "heff_applications": 2108, "published": bench.N2_PUBLISHED, "speedup_vs_published": 14.4},
+    }
+    line = bench.json.dumps(bench.summary(out))
+    assert len(line) < 2000
+    got = bench.json.loads(line)
+    for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+              "vs_baseline", "dtype", "data", "config"):
+        assert got[k] == out[k]
+    assert got["sweep"]["fp64"]["seconds"] == sweep["seconds"]
+    # parts that a run left out
+    short = dict(out, roofline=bench.roofline_record(1e11, 1e9, 10.0, None, None), cpu_baseline=None,
+                 n2_ccpvdz_published_point=None, sweep={"fp64": sweep})
+    assert "cpu_baseline" not in bench.summary(short) and bench.summary(short)["value"] == 17.1234
