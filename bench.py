@@ -141,7 +141,7 @@ def traffic_numbers(fetch_csv, write_csv, steps):
     rd = sum(fk) * fscale * 1024.0 / steps
     wr = sum(wk) * wscale * 1024.0 / steps
     out = {
-        "kernel": "every kernel of one Heff application (k_bspmv, k_tiles_stream1, k_tiles_wave1, k_tiles_wave2, "
+        "kernel": "every kernel of one Heff application (k_bspmv, k_strips, k_tiles_stream1, k_tiles_wave1, k_tiles_wave2, "
                   "k_tiles_fit, k_fchain, k_chain and their reductions)",
         "workload": "Heff x at sites 15-16 of the warmed-up L=32 D=2000 random D2h state",
         "bytes_per_launch": rd + wr, "read_bytes": rd, "write_bytes": wr,

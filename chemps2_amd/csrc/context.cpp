@@ -828,8 +828,10 @@ void Ctx::prepare(int st) {
   // input share W (a carries over to phase 2): at the L = 32, D = 2000 middle site 1.60 M
   // terms then have 1.23 M W of 4.4 GB instead of 1.60 M of 9.2 GB, and take 97 instead of
   // 142 GF; 16.1 -> 12.6 ms a product. A short list keeps the reference's order and one W
-  // (with a) per term: launches and latency bound its product (402 against 382 us at 42 k
-  // terms, 383 against 362 us at 30 k), and its rounding stays that of the reference's order.
+  // (with a) per term. Sharing is 3 to 9 % faster there too (402 -> 382 us at 42 k terms,
+  // 383 -> 362 us at 30 k), but its launches and latency leave little to gain, and another
+  // rounding moves the number of iterations of the Davidson solves on such lists by a fifth
+  // either way.
   DevTile1* t1 = nullptr;      // the device records, built in page-locked staging
   DevGemmOp* o2 = nullptr;
   DevTile* t2 = nullptr;

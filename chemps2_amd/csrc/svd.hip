@@ -18,10 +18,10 @@
 // the test that ends the sweeps (no entry above the rounding floor) is on fresh ones.
 //
 // Measured on the MI355X (Split and Join of one site): 196 sectors of up to 147 columns
-// (L = 32, D = 2000, D2h) 3.8 ms, where one workgroup per sector rotating columns in global
-// memory took 33 ms; 69 sectors of up to 615 columns (no point group, D = 2000) 19.8 ms,
-// where those above 256 went to rocSOLVER's dgesvdj (930 ms). The reconstructed object is
-// 2.8e-14 (wide: 1.6e-13) from LAPACK's, the old paths' 3.1e-14 (2.2e-13).
+// (L = 32, D = 2000, D2h) 3.7 ms, where one workgroup per sector rotating columns in global
+// memory took 33 ms; 69 sectors of up to 615 columns (no point group, D = 2000) 20.2 ms,
+// where those above 256 went to rocSOLVER's dgesvdj (930 ms). The re-joined object is 2.8e-15
+// (wide: 6.0e-15) from LAPACK's, those paths' 3.1e-14 (2.2e-13).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
